@@ -65,8 +65,9 @@ extern "C" {
                                           (adam.py:538-543); every row needs max_exp_avg_sq */
 
 /* mi_adamw_tensor.flags */
-#define MI_ADAMW_T_VEC (1 << 0) /* fp32 pointers 16-byte aligned and bf16 pointers 8-byte
-                                   aligned: the dwordx4 path may be used */
+#define MI_ADAMW_T_VEC (1 << 0) /* promises fp32 pointers 16-byte aligned and bf16 pointers
+                                   8-byte aligned (the flat entry points check it); the
+                                   kernels take four elements at a time with or without it */
 
 typedef struct mi_adamw_tensor {
     float *param;          /* fp32 master parameter, updated in place                */
