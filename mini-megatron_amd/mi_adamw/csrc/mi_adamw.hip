@@ -56,10 +56,7 @@ constexpr int kVec = 4;                       // fp32 elements per lane per acce
 // 4096-element chunk, so a workgroup has four dwordx4 loads per lane in flight.
 constexpr int kNormThreads = 256;
 constexpr int kNormTile = kNormThreads * kVec;
-// Update: 1024-thread workgroups (16 wave64), one 4096-element tile per chunk.
-// Measured on MI355X: a whole chunk per tile (each workgroup issues all its
-// loads at once and retires) streams 3-4% faster than 256-thread workgroups
-// looping over four tiles.
+// Scale and widen: 1024-thread workgroups (16 wave64), one 4096-element tile per chunk.
 constexpr int kUpdThreads = 1024;
 constexpr int kUpdTile = kUpdThreads * kVec;
 constexpr int kChunkQuantum = kUpdTile;       // chunk sizes are multiples of this
@@ -159,8 +156,8 @@ __device__ __forceinline__ void adamw_elem(float& p, float g, float& m, float& v
 // gives the division's bits; without it, by the division itself.  The host-step chain
 // and the per-row chain (FusedRowsHyper) take kRecip: their per-step values are kernel
 // arguments or scalar loads, so the reciprocal costs no vector register.  The device-step
-// chain that forms them in every workgroup does so after two out-of-line pow calls with
-// the first tile's loads in flight, where one more value spills, so it divides.
+// chain that forms them in every wave does so after two out-of-line pow calls with the
+// tile's loads in flight, and divides.
 template <bool kRecip>
 struct FusedScalarsT {
     double beta1, one_minus_beta1;
@@ -476,8 +473,7 @@ struct FusedPack {
     FusedSet h[MI_ADAMW_MAX_HYPER];
 };
 
-// pow in float64, out of line: inlined into the update it adds 10-15 VGPRs to every
-// instance of the device-step chain.
+// pow in float64, out of line: one copy for every instance of the device-step chain.
 __device__ __attribute__((noinline)) double pow_f64(double x, double y) { return pow(x, y); }
 
 // torch's fused=True chain: the per-step values of fused_adam_utils.cuh
@@ -494,9 +490,7 @@ struct FusedHyper {
     static constexpr bool kCapt = false;
     static constexpr bool kLate = true;
     static constexpr bool kProbe = false;
-    // every wave forms its own: with device step counts the two out-of-line float64 pow
-    // calls in one wave's branch spill under this chain's 64-VGPR cap, and with host step
-    // counts the prologue is a few loads
+    // every wave forms its own: with host step counts that is a few loads
     static constexpr bool kShare = false;
     FusedPack fp;
     const float* steps;
@@ -799,11 +793,26 @@ __global__ __launch_bounds__(kNormThreads) void mi_adamw_sumsq_reduce_kernel(
 // ---------------------------------------------------------------------------
 // Pass 2: the AdamW update.
 //
-// One chunk per workgroup (grid = number of chunks): the hardware dispatcher
-// hands the next chunk to whichever CU frees a slot, which balances ragged
-// tensors.  With the default 4096-element chunk a workgroup covers its chunk in
-// one tile.  Larger chunks are walked tile by tile, software-pipelined: the
-// loads of tile k+1 are issued before tile k is computed and stored.
+// A work item is one tile of a chunk, kThreads * 4 elements, one dwordx4 group per lane:
+// every lane issues its four loads at once, and the hardware dispatcher hands the next
+// item to whichever CU frees a slot, which balances ragged tensors.  The step moves 22-34
+// bytes for ~15 operations per element, so what bounds it is how HBM takes the mix of
+// four read and three or four written streams, and that depends on two things:
+//   - how much is in flight.  1024 threads per CU (4 wave64 per SIMD) and not the 2048
+//     that fit: beyond that the lines in flight on an XCD approach its 4 MB L2 and are
+//     written back out of order.
+//   - which XCD touches what.  Workgroups go to the 8 XCDs in turn, so in plain order each
+//     XCD touches every eighth tile of every stream; item_order gives it runs of 128
+//     tiles (128K elements) instead.
+// The memory traffic alone (no arithmetic, mean of 12 sets of buffers as allocated, 22 and
+// 30 bytes per element), GB/s: 5,640 with 2048 threads per CU in plain order, 5,820 with
+// half of them, 5,730 with runs alone, 6,350 with both.  256-thread workgroups (four per
+// CU) spread less over the buffers' places than one of 1024 (6,190-6,510 against
+// 6,030-6,500); 3 or 5 of them 6,290 and 6,240; a persistent grid 5,100-5,500.
+// The step on buffers as allocated, before (1024-thread workgroups over 4096 elements, two
+// per CU, plain order) and now: 1.4G parameters, bf16 moments, flat, clip + copy 6,272 ->
+// 5,713 us; gpt-125m tables, clip 857 -> 797, fused=True chain without the clip 801 -> 717;
+// on buffers placed by measured trials 35.49 -> 35.19 ms at 6.9G parameters.
 
 template <typename StateT, bool kAms>
 struct Tile {
@@ -818,13 +827,25 @@ struct Tile {
     }
 };
 
-// Waves per SIMD each instance must allow: 8 (two workgroups per CU, at most 64 VGPRs)
-// for the fused=True chain's instances without amsgrad, whose float64 math would
-// otherwise take 65-70 VGPRs and halve the workgroups in flight; 4 (one workgroup,
-// what 1024-thread workgroups need anyway) for the rest.
-template <class HS, bool kAms>
-constexpr int update_waves_per_eu() {
-    return (HS::kLate && !HS::kCapt && !kAms) ? 8 : 4;
+// Lanes of an instance's workgroups.  The chains whose first wave forms the per-step
+// values for the whole workgroup (kShare: a few hundred instructions) take the widest
+// workgroup, so that they are formed least often.
+template <class HS>
+constexpr int update_threads() {
+    return HS::kShare ? 1024 : 256;
+}
+
+// The item that workgroup index w takes: in every full group of 8 runs, XCD w % 8 gets one
+// contiguous run, another one from group to group (a fixed one leaves some placements of
+// the buffers 3% slower).
+constexpr int kRunTiles = 128;
+__device__ __forceinline__ int64_t item_order(int64_t w, int64_t n_items) {
+    constexpr int64_t kGroup = 8 * kRunTiles;
+    static_assert(kGroup == 1 << 10, "the shift below");
+    const int64_t base = w & ~(kGroup - 1);
+    if (base + kGroup > n_items) return w;
+    const int64_t r = w - base;
+    return base + ((r ^ (w >> 10)) & 7) * kRunTiles + (r >> 3);
 }
 
 // The scalars of a chunk formed by the workgroup's first wave and read by every wave
@@ -858,25 +879,33 @@ __device__ __forceinline__ typename HS::Scalars shared_scalars(const HS& hs,
 }
 
 template <class Src, class HS, typename StateT, bool kClip, bool kCopy, bool kWriteGrad, bool kAms>
-__global__ __launch_bounds__(kUpdThreads)
-__attribute__((amdgpu_waves_per_eu(update_waves_per_eu<HS, kAms>())))
+__global__ __launch_bounds__(update_threads<HS>())
+__attribute__((amdgpu_waves_per_eu(4, 4)))   // the cap above, and 128 VGPRs per lane
 void mi_adamw_update_kernel(
-    Src src, int64_t n_chunks, int64_t chunk_elems, HS hs,
+    Src src, int64_t n_items, int64_t chunk_elems, int32_t tiles, int32_t tiles_shift, HS hs,
     const float* __restrict__ grad_scale, float pre) {
     using IO = StateIO<StateT>;
     using T = Tile<StateT, kAms>;
+    constexpr int kThreads = update_threads<HS>();
+    constexpr int kTile = kThreads * kVec;
     constexpr bool kCapt = HS::kCapt;
     constexpr bool kLate = HS::kLate;
     constexpr bool kProbe = HS::kProbe;
     const float scale = kClip ? *grad_scale : 1.0f;
-    int parity = 0;   // shared_scalars' buffer of this chunk
-    for (int64_t c = blockIdx.x; c < n_chunks; c += gridDim.x) {
+    int parity = 0;   // shared_scalars' buffer of this item
+    for (int64_t w = blockIdx.x; w < n_items; w += gridDim.x) {
+        // chunk and tile of the item (tiles per chunk: 4 at the default chunk size)
+        const int64_t it = item_order(w, n_items);
+        const int64_t c = tiles_shift >= 0 ? it >> tiles_shift : it / tiles;
         mi_adamw_tensor t;
         int64_t begin, end;
         int32_t row;
         src.get(c, chunk_elems, t, begin, end, row);
+        begin += (it - c * tiles) * kTile;
+        if (begin >= end) continue;                // past the tensor's last, shorter chunk
+        if (end > begin + kTile) end = begin + kTile;
         // Default chain: the scalars are kernel arguments.  Capturable and fused
-        // chains: they are formed once the first tile's loads are in flight; in the
+        // chains: they are formed once the tile's loads are in flight; in the
         // capturable chain (two powf, three divisions: a few hundred instructions) by
         // the first wave alone and shared through LDS (kShare).
         typename HS::Scalars h;
@@ -889,9 +918,9 @@ void mi_adamw_update_kernel(
         void* __restrict__ X = t.max_exp_avg_sq;
 
         const int64_t vend = begin + ((end - begin) & ~static_cast<int64_t>(kVec - 1));
-        int64_t i = begin + threadIdx.x * kVec;
-        T cur;
+        const int64_t i = begin + threadIdx.x * kVec;
         const bool have = i < vend;
+        T cur;
         if (have) cur.load(P, G, M, V, X, i);
         if (kLate) {
             __builtin_amdgcn_sched_barrier(0);
@@ -902,36 +931,26 @@ void mi_adamw_update_kernel(
                 h = hs.get(t, row);
             }
         }
+        const float gmul = h.grad_sign;
         if (have) {
-            const float gmul = h.grad_sign;
-            while (true) {
-                const int64_t j = i + kUpdTile;
-                const bool more = j < vend;
-                T nxt = cur;
-                if (more) nxt.load(P, G, M, V, X, j);
-                // the stored value of div_(world), then of the clip, then -g with maximize
-                f32x4 gs = f32x4{cur.g.x * pre, cur.g.y * pre, cur.g.z * pre, cur.g.w * pre};
-                if (kClip) gs = f32x4{gs.x * scale, gs.y * scale, gs.z * scale, gs.w * scale};
-                if (kWriteGrad) st4(G + i, gs);
-                if (kProbe) {
-                    keep(gs);
-                } else {
-                    gs = f32x4{gs.x * gmul, gs.y * gmul, gs.z * gmul, gs.w * gmul};
-                    adamw_vec<kAms, kCapt>(cur.p, gs, cur.m, cur.v, cur.x, h);
-                }
-                st4(P + i, cur.p);
-                IO::st(M, i, cur.m);
-                IO::st(V, i, cur.v);
-                if (kAms) IO::st(X, i, cur.x);
-                if (kCopy) st4_bf16(C + i, cur.p);
-                if (!more) break;
-                cur = nxt;
-                i = j;
+            // the stored value of div_(world), then of the clip, then -g with maximize
+            f32x4 gs = f32x4{cur.g.x * pre, cur.g.y * pre, cur.g.z * pre, cur.g.w * pre};
+            if (kClip) gs = f32x4{gs.x * scale, gs.y * scale, gs.z * scale, gs.w * scale};
+            if (kWriteGrad) st4(G + i, gs);
+            if (kProbe) {
+                keep(gs);
+            } else {
+                gs = f32x4{gs.x * gmul, gs.y * gmul, gs.z * gmul, gs.w * gmul};
+                adamw_vec<kAms, kCapt>(cur.p, gs, cur.m, cur.v, cur.x, h);
             }
+            st4(P + i, cur.p);
+            IO::st(M, i, cur.m);
+            IO::st(V, i, cur.v);
+            if (kAms) IO::st(X, i, cur.x);
+            if (kCopy) st4_bf16(C + i, cur.p);
         }
         // the tensor's last elements, up to three
-        const float gmul = h.grad_sign;
-        for (int64_t j = vend + threadIdx.x; j < end; j += kUpdThreads) {
+        for (int64_t j = vend + threadIdx.x; j < end; j += kThreads) {
             float g1 = ld1(G + j) * pre;
             if (kClip) g1 = g1 * scale;
             if (kWriteGrad) st1(G + j, g1);
@@ -1100,17 +1119,22 @@ int launch_sumsq_total(const Src& src, int64_t n_chunks, int64_t chunk_elems, fl
 template <class Src, class HS, typename StateT, bool kClip, bool kCopy, bool kWriteGrad,
           bool kAms>
 int launch_update_k(const Src& src, int64_t n_chunks, int64_t chunk_elems, const HS& hs,
-                    const float* scale, float pre, unsigned grid, hipStream_t s) {
+                    const float* scale, float pre, int32_t max_blocks, hipStream_t s) {
+    constexpr int kThreads = update_threads<HS>();
+    const int32_t tiles = static_cast<int32_t>(chunk_elems / (kThreads * kVec));
+    const int32_t shift = (tiles & (tiles - 1)) == 0 ? __builtin_ctz(tiles) : -1;
+    if (n_chunks > INT64_MAX / tiles) return MI_ADAMW_E_INVALID;
+    const int64_t n_items = n_chunks * tiles;
     hipLaunchKernelGGL((mi_adamw_update_kernel<Src, HS, StateT, kClip, kCopy, kWriteGrad, kAms>),
-                       dim3(grid), dim3(kUpdThreads), 0, s, src, n_chunks, chunk_elems, hs, scale,
-                       pre);
+                       dim3(grid_for(n_items, max_blocks, kThreads)), dim3(kThreads), 0, s, src,
+                       n_items, chunk_elems, tiles, shift, hs, scale, pre);
     return launch_status();
 }
 
 // Runtime flags -> kernel template: one instantiation per (copy, write-grad, amsgrad).
 template <class Src, class HS, typename StateT, bool kClip>
 int launch_update_cw(const Src& src, int64_t n_chunks, int64_t chunk_elems, const HS& hs,
-                     const float* scale, float pre, int32_t flags, unsigned grid,
+                     const float* scale, float pre, int32_t flags, int32_t max_blocks,
                      hipStream_t s) {
     const int sel = ((flags & MI_ADAMW_F_BF16_COPY) ? 1 : 0) |
                     ((flags & MI_ADAMW_F_WRITE_GRAD) ? 2 : 0) |
@@ -1118,7 +1142,7 @@ int launch_update_cw(const Src& src, int64_t n_chunks, int64_t chunk_elems, cons
 #define MI_ADAMW_SEL(k, C, W, A)                                                              \
     case k:                                                                                   \
         return launch_update_k<Src, HS, StateT, kClip, C, W, A>(src, n_chunks, chunk_elems,  \
-                                                                 hs, scale, pre, grid, s);
+                                                                 hs, scale, pre, max_blocks, s);
     switch (sel) {
         MI_ADAMW_SEL(0, false, false, false)
         MI_ADAMW_SEL(1, true, false, false)
@@ -1145,16 +1169,15 @@ int launch_update(const Src& src, int64_t n_chunks, int64_t chunk_elems, const H
         return MI_ADAMW_E_INVALID;
     const bool clip = flags & MI_ADAMW_F_CLIP;
     if (clip && !scale) return MI_ADAMW_E_INVALID;
-    const unsigned grid = grid_for(n_chunks, max_blocks, kUpdThreads);
     if (state_dtype == MI_ADAMW_STATE_F32)
         return clip ? launch_update_cw<Src, HS, float, true>(src, n_chunks, chunk_elems, hs,
-                                                              scale, pre, flags, grid, s)
+                                                              scale, pre, flags, max_blocks, s)
                     : launch_update_cw<Src, HS, float, false>(src, n_chunks, chunk_elems, hs,
-                                                               scale, pre, flags, grid, s);
+                                                               scale, pre, flags, max_blocks, s);
     return clip ? launch_update_cw<Src, HS, uint16_t, true>(src, n_chunks, chunk_elems, hs, scale,
-                                                             pre, flags, grid, s)
+                                                             pre, flags, max_blocks, s)
                 : launch_update_cw<Src, HS, uint16_t, false>(src, n_chunks, chunk_elems, hs,
-                                                              scale, pre, flags, grid, s);
+                                                              scale, pre, flags, max_blocks, s);
 }
 
 // The memory-only twin of launch_update (no clip: the gradient is read either way).
@@ -1167,13 +1190,12 @@ int launch_probe(const Src& src, int64_t n_chunks, int64_t chunk_elems, int32_t 
     flags &= ~MI_ADAMW_F_CLIP;
     if (flags & ~(MI_ADAMW_F_BF16_COPY | MI_ADAMW_F_WRITE_GRAD | MI_ADAMW_F_AMSGRAD))
         return MI_ADAMW_E_INVALID;
-    const unsigned grid = grid_for(n_chunks, max_blocks, kUpdThreads);
     const ProbeHyper hs;
     if (state_dtype == MI_ADAMW_STATE_F32)
         return launch_update_cw<Src, ProbeHyper, float, false>(src, n_chunks, chunk_elems, hs,
-                                                               nullptr, 1.0f, flags, grid, s);
+                                                               nullptr, 1.0f, flags, max_blocks, s);
     return launch_update_cw<Src, ProbeHyper, uint16_t, false>(src, n_chunks, chunk_elems, hs,
-                                                              nullptr, 1.0f, flags, grid, s);
+                                                              nullptr, 1.0f, flags, max_blocks, s);
 }
 
 // The kernel's form of one mi_adamw_fused_hyper.  With host step counts the per-step
