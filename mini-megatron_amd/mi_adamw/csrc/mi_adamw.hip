@@ -56,10 +56,7 @@ constexpr int kVec = 4;                       // fp32 elements per lane per acce
 // 4096-element chunk, so a workgroup has four dwordx4 loads per lane in flight.
 constexpr int kNormThreads = 256;
 constexpr int kNormTile = kNormThreads * kVec;
-// Scale and widen: 1024-thread workgroups (16 wave64), one 4096-element tile per chunk.
-constexpr int kUpdThreads = 1024;
-constexpr int kUpdTile = kUpdThreads * kVec;
-constexpr int kChunkQuantum = kUpdTile;       // chunk sizes are multiples of this
+constexpr int kChunkQuantum = 4096;           // chunk sizes are multiples of this
 static_assert(kChunkQuantum == MI_ADAMW_CHUNK_QUANTUM, "header and kernels agree");
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
@@ -791,6 +788,42 @@ __global__ __launch_bounds__(kNormThreads) void mi_adamw_sumsq_reduce_kernel(
 }
 
 // ---------------------------------------------------------------------------
+// Work items of the streaming passes (update, scale, widen): one tile of a chunk each.
+
+// The item that workgroup index w takes: in every full group of 8 runs of kRun items, XCD
+// w % 8 gets one contiguous run, another one from group to group (a fixed one leaves some
+// placements of the update's buffers 3% slower).
+template <int kRun>
+__device__ __forceinline__ int64_t item_order(int64_t w, int64_t n_items) {
+    static_assert((kRun & (kRun - 1)) == 0, "masks and shifts below");
+    constexpr int64_t kGroup = 8 * kRun;
+    const int64_t base = w & ~(kGroup - 1);
+    if (base + kGroup > n_items) return w;
+    const int64_t r = w - base;
+    return base + ((r ^ (w >> __builtin_ctzll(kGroup))) & 7) * kRun + (r >> 3);
+}
+
+// The items of a launch: chunks of chunk_elems elements, `tiles` tiles each.
+struct Items {
+    int64_t n;
+    int64_t chunk_elems;
+    int32_t tiles;
+    int32_t shift;    // log2(tiles), or -1
+    // Item `it`: its chunk's tensor and row, and the tile's elements.  False past the end of
+    // the tensor's last, shorter chunk.
+    template <int kTile, class Src>
+    __device__ __forceinline__ bool get(const Src& src, int64_t it, mi_adamw_tensor& t,
+                                        int64_t& begin, int64_t& end, int32_t& row) const {
+        const int64_t c = shift >= 0 ? it >> shift : it / tiles;
+        src.get(c, chunk_elems, t, begin, end, row);
+        begin += (it - c * tiles) * kTile;
+        if (begin >= end) return false;
+        if (end > begin + kTile) end = begin + kTile;
+        return true;
+    }
+};
+
+// ---------------------------------------------------------------------------
 // Pass 2: the AdamW update.
 //
 // A work item is one tile of a chunk, kThreads * 4 elements, one dwordx4 group per lane:
@@ -827,25 +860,14 @@ struct Tile {
     }
 };
 
+constexpr int kUpdRun = 128;
+
 // Lanes of an instance's workgroups.  The chains whose first wave forms the per-step
 // values for the whole workgroup (kShare: a few hundred instructions) take the widest
 // workgroup, so that they are formed least often.
 template <class HS>
 constexpr int update_threads() {
     return HS::kShare ? 1024 : 256;
-}
-
-// The item that workgroup index w takes: in every full group of 8 runs, XCD w % 8 gets one
-// contiguous run, another one from group to group (a fixed one leaves some placements of
-// the buffers 3% slower).
-constexpr int kRunTiles = 128;
-__device__ __forceinline__ int64_t item_order(int64_t w, int64_t n_items) {
-    constexpr int64_t kGroup = 8 * kRunTiles;
-    static_assert(kGroup == 1 << 10, "the shift below");
-    const int64_t base = w & ~(kGroup - 1);
-    if (base + kGroup > n_items) return w;
-    const int64_t r = w - base;
-    return base + ((r ^ (w >> 10)) & 7) * kRunTiles + (r >> 3);
 }
 
 // The scalars of a chunk formed by the workgroup's first wave and read by every wave
@@ -882,8 +904,7 @@ template <class Src, class HS, typename StateT, bool kClip, bool kCopy, bool kWr
 __global__ __launch_bounds__(update_threads<HS>())
 __attribute__((amdgpu_waves_per_eu(4, 4)))   // the cap above, and 128 VGPRs per lane
 void mi_adamw_update_kernel(
-    Src src, int64_t n_items, int64_t chunk_elems, int32_t tiles, int32_t tiles_shift, HS hs,
-    const float* __restrict__ grad_scale, float pre) {
+    Src src, Items items, HS hs, const float* __restrict__ grad_scale, float pre) {
     using IO = StateIO<StateT>;
     using T = Tile<StateT, kAms>;
     constexpr int kThreads = update_threads<HS>();
@@ -893,17 +914,11 @@ void mi_adamw_update_kernel(
     constexpr bool kProbe = HS::kProbe;
     const float scale = kClip ? *grad_scale : 1.0f;
     int parity = 0;   // shared_scalars' buffer of this item
-    for (int64_t w = blockIdx.x; w < n_items; w += gridDim.x) {
-        // chunk and tile of the item (tiles per chunk: 4 at the default chunk size)
-        const int64_t it = item_order(w, n_items);
-        const int64_t c = tiles_shift >= 0 ? it >> tiles_shift : it / tiles;
+    for (int64_t w = blockIdx.x; w < items.n; w += gridDim.x) {
         mi_adamw_tensor t;
         int64_t begin, end;
         int32_t row;
-        src.get(c, chunk_elems, t, begin, end, row);
-        begin += (it - c * tiles) * kTile;
-        if (begin >= end) continue;                // past the tensor's last, shorter chunk
-        if (end > begin + kTile) end = begin + kTile;
+        if (!items.get<kTile>(src, item_order<kUpdRun>(w, items.n), t, begin, end, row)) continue;
         // Default chain: the scalars are kernel arguments.  Capturable and fused
         // chains: they are formed once the tile's loads are in flight; in the
         // capturable chain (two powf, three divisions: a few hundred instructions) by
@@ -972,43 +987,59 @@ void mi_adamw_update_kernel(
 
 // ---------------------------------------------------------------------------
 // g *= coef (clip write-back on its own).
+//
+// One stream read and written: one dwordx4 group per lane, 512-thread workgroups, as many
+// as fit (the table lookup's latency needs them: with six waves per SIMD it is 5% slower),
+// runs of 32 tiles per XCD.  clip_grad_norm_ of 163M gradients, 1024-thread workgroups over
+// 4096 elements in plain order 309 us, in runs of 16 301, this 300; four groups per lane
+// 314-380.  Stores that stay in the caches end the pass 5% sooner but the next pass pays
+// for them (330 us a call).
 
-__global__ __launch_bounds__(kUpdThreads) void mi_adamw_scale_kernel(
-    TableSource src, int64_t n_chunks, int64_t chunk_elems, const float* __restrict__ coef) {
+constexpr int kScaleThreads = 512;
+constexpr int kScaleTile = kScaleThreads * kVec;
+constexpr int kScaleRun = 32;
+
+__global__ __launch_bounds__(kScaleThreads) void mi_adamw_scale_kernel(
+    TableSource src, Items items, const float* __restrict__ coef) {
     const float s = *coef;
-    for (int64_t c = blockIdx.x; c < n_chunks; c += gridDim.x) {
+    for (int64_t w = blockIdx.x; w < items.n; w += gridDim.x) {
         mi_adamw_tensor t;
         int64_t begin, end;
         int32_t row;
-        src.get(c, chunk_elems, t, begin, end, row);
+        if (!items.get<kScaleTile>(src, item_order<kScaleRun>(w, items.n), t, begin, end, row))
+            continue;
         float* __restrict__ G = t.grad;
         const int64_t vend = begin + ((end - begin) & ~static_cast<int64_t>(kVec - 1));
-        for (int64_t i = begin + threadIdx.x * kVec; i < vend; i += kUpdTile) {
-            f32x4 g = ld4(G + i);
+        const int64_t i = begin + threadIdx.x * kVec;
+        if (i < vend) {
+            const f32x4 g = ld4(G + i);
             st4(G + i, f32x4{g.x * s, g.y * s, g.z * s, g.w * s});
         }
-        for (int64_t j = vend + threadIdx.x; j < end; j += kUpdThreads) st1(G + j, ld1(G + j) * s);
+        const int64_t j = vend + threadIdx.x;      // the tensor's last elements, up to three
+        if (j < end) st1(G + j, ld1(G + j) * s);
     }
 }
 
 // ---------------------------------------------------------------------------
 // bf16 -> fp32 of every tensor of the tables: param = (float)param_copy, exact (the bf16
-// bits are the upper half of the fp32 value, NaN payloads included).
+// bits are the upper half of the fp32 value, NaN payloads included).  Items as in
+// the scale pass.
 
-__global__ __launch_bounds__(kUpdThreads) void mi_adamw_widen_kernel(
-    TableSource src, int64_t n_chunks, int64_t chunk_elems) {
-    for (int64_t c = blockIdx.x; c < n_chunks; c += gridDim.x) {
+__global__ __launch_bounds__(kScaleThreads) void mi_adamw_widen_kernel(TableSource src,
+                                                                       Items items) {
+    for (int64_t w = blockIdx.x; w < items.n; w += gridDim.x) {
         mi_adamw_tensor t;
         int64_t begin, end;
         int32_t row;
-        src.get(c, chunk_elems, t, begin, end, row);
+        if (!items.get<kScaleTile>(src, item_order<kScaleRun>(w, items.n), t, begin, end, row))
+            continue;
         const uint16_t* __restrict__ S = t.param_copy;
         float* __restrict__ D = t.param;
         const int64_t vend = begin + ((end - begin) & ~static_cast<int64_t>(kVec - 1));
-        for (int64_t i = begin + threadIdx.x * kVec; i < vend; i += kUpdTile)
-            st4(D + i, ld4_bf16(S + i));
-        for (int64_t j = vend + threadIdx.x; j < end; j += kUpdThreads)
-            st1(D + j, bf16_to_f32(ld1_u16(S + j)));
+        const int64_t i = begin + threadIdx.x * kVec;
+        if (i < vend) st4(D + i, ld4_bf16(S + i));
+        const int64_t j = vend + threadIdx.x;
+        if (j < end) st1(D + j, bf16_to_f32(ld1_u16(S + j)));
     }
 }
 
@@ -1068,6 +1099,14 @@ unsigned grid_for(int64_t n_chunks, int32_t max_blocks, int threads) {
     return static_cast<unsigned>(g);
 }
 
+// The tiles of n_chunks chunks (chunk sizes are multiples of kChunkQuantum, of which every
+// tile size is a divisor).
+Items items_of(int64_t n_chunks, int64_t chunk_elems, int tile) {
+    const int32_t tiles = static_cast<int32_t>(chunk_elems / tile);
+    const int32_t shift = (tiles & (tiles - 1)) == 0 ? __builtin_ctz(tiles) : -1;
+    return Items{n_chunks * tiles, chunk_elems, tiles, shift};
+}
+
 bool aligned(const void* p, uintptr_t a) { return (reinterpret_cast<uintptr_t>(p) & (a - 1)) == 0; }
 
 bool finite(float x) { return x - x == 0.0f; }
@@ -1121,13 +1160,10 @@ template <class Src, class HS, typename StateT, bool kClip, bool kCopy, bool kWr
 int launch_update_k(const Src& src, int64_t n_chunks, int64_t chunk_elems, const HS& hs,
                     const float* scale, float pre, int32_t max_blocks, hipStream_t s) {
     constexpr int kThreads = update_threads<HS>();
-    const int32_t tiles = static_cast<int32_t>(chunk_elems / (kThreads * kVec));
-    const int32_t shift = (tiles & (tiles - 1)) == 0 ? __builtin_ctz(tiles) : -1;
-    if (n_chunks > INT64_MAX / tiles) return MI_ADAMW_E_INVALID;
-    const int64_t n_items = n_chunks * tiles;
+    const Items items = items_of(n_chunks, chunk_elems, kThreads * kVec);
     hipLaunchKernelGGL((mi_adamw_update_kernel<Src, HS, StateT, kClip, kCopy, kWriteGrad, kAms>),
-                       dim3(grid_for(n_items, max_blocks, kThreads)), dim3(kThreads), 0, s, src,
-                       n_items, chunk_elems, tiles, shift, hs, scale, pre);
+                       dim3(grid_for(items.n, max_blocks, kThreads)), dim3(kThreads), 0, s, src,
+                       items, hs, scale, pre);
     return launch_status();
 }
 
@@ -1465,9 +1501,9 @@ int mi_adamw_scale_grads(const mi_adamw_tensor* d_tensors, const mi_adamw_chunk*
     if (!d_tensors || !d_chunks || !d_coef || n_chunks <= 0 || !chunk_elems_ok(chunk_elems))
         return MI_ADAMW_E_INVALID;
     TableSource src{d_tensors, d_chunks};
-    hipLaunchKernelGGL(mi_adamw_scale_kernel, dim3(grid_for(n_chunks, 0, kUpdThreads)),
-                       dim3(kUpdThreads), 0,
-                       static_cast<hipStream_t>(stream), src, n_chunks, chunk_elems, d_coef);
+    const Items items = items_of(n_chunks, chunk_elems, kScaleTile);
+    hipLaunchKernelGGL(mi_adamw_scale_kernel, dim3(grid_for(items.n, 0, kScaleThreads)), dim3(kScaleThreads), 0,
+                       static_cast<hipStream_t>(stream), src, items, d_coef);
     return launch_status();
 }
 
@@ -1476,9 +1512,9 @@ int mi_adamw_widen_bf16(const mi_adamw_tensor* d_tensors, const mi_adamw_chunk* 
     if (!d_tensors || !d_chunks || n_chunks <= 0 || !chunk_elems_ok(chunk_elems))
         return MI_ADAMW_E_INVALID;
     TableSource src{d_tensors, d_chunks};
-    hipLaunchKernelGGL(mi_adamw_widen_kernel, dim3(grid_for(n_chunks, 0, kUpdThreads)),
-                       dim3(kUpdThreads), 0, static_cast<hipStream_t>(stream), src, n_chunks,
-                       chunk_elems);
+    const Items items = items_of(n_chunks, chunk_elems, kScaleTile);
+    hipLaunchKernelGGL(mi_adamw_widen_kernel, dim3(grid_for(items.n, 0, kScaleThreads)), dim3(kScaleThreads), 0,
+                       static_cast<hipStream_t>(stream), src, items);
     return launch_status();
 }
 
