@@ -64,6 +64,10 @@ extern "C" {
                                           exp_avg_sq), and the denominator is taken from it
                                           (adam.py:538-543); every row needs max_exp_avg_sq */
 
+#define MI_ADAMW_F_NORM_BLOCK (1 << 4) /* with MI_ADAMW_F_CLIP: d_grad_scale points to a
+                                          mi_adamw_norm_block (cast to const float *) that
+                                          mi_adamw_grad_norm_block* wrote earlier on the stream */
+
 /* mi_adamw_tensor.flags */
 #define MI_ADAMW_T_VEC (1 << 0) /* promises fp32 pointers 16-byte aligned and bf16 pointers
                                    8-byte aligned (the flat entry points check it); the
@@ -194,6 +198,33 @@ int mi_adamw_grad_norm(const mi_adamw_tensor *d_tensors, const mi_adamw_chunk *d
 /* Same over one contiguous fp32 gradient range of n elements. */
 int mi_adamw_grad_norm_flat(const float *d_grad, int64_t n, int64_t chunk_elems, float max_norm,
                             double *d_partials, float *d_norm, float *d_coef, void *stream);
+
+/* Device memory that carries a clip from its norm pass to its update.  The caller allocates
+ * it (MI_ADAMW_NORM_BLOCK_BYTES, 64-byte aligned); its contents are the library's. */
+#define MI_ADAMW_NORM_BLOCK_PARTIALS 512
+typedef struct mi_adamw_norm_block {
+    double partials[MI_ADAMW_NORM_BLOCK_PARTIALS]; /* the norm pass's partial sums         */
+    float *norm;                                   /* where the norm goes                  */
+    float max_norm;
+    int32_t n_partials;                            /* 0: coef is final                     */
+    float coef;
+    float reserved[11];
+} mi_adamw_norm_block;
+#define MI_ADAMW_NORM_BLOCK_BYTES 4160
+
+/* mi_adamw_grad_norm with its second launch left to the update: the sum-of-squares pass
+ * over grad_prescale * g into *d_block, and the norm and coefficient, the same bits, formed
+ * by the update launched next on the stream with MI_ADAMW_F_CLIP | MI_ADAMW_F_NORM_BLOCK and
+ * d_grad_scale = (const float *)d_block.  *d_norm is written by then.  Sets too large to
+ * gain from that (every workgroup of the update would reduce the partial sums again) have
+ * both launched here; the caller's calls are the same. */
+int mi_adamw_grad_norm_block(const mi_adamw_tensor *d_tensors, const mi_adamw_chunk *d_chunks,
+                             int64_t n_chunks, int64_t chunk_elems, float grad_prescale,
+                             float max_norm, mi_adamw_norm_block *d_block, float *d_norm,
+                             void *stream);
+int mi_adamw_grad_norm_block_flat(const float *d_grad, int64_t n, int64_t chunk_elems,
+                                  float grad_prescale, float max_norm,
+                                  mi_adamw_norm_block *d_block, float *d_norm, void *stream);
 
 /* Bytes of device scratch that mi_adamw_grad_norm_flat_noalloc uses on each GPU: one
  * float64 partial sum per workgroup of the norm pass, which never runs more than 512. */

@@ -29,6 +29,7 @@ ABI_VERSION = 9
 MAX_HYPER = 16
 MAX_NORM_BLOCKS = 4096
 NOALLOC_SCRATCH_BYTES = 4096
+NORM_BLOCK_BYTES = 4160   # one mi_adamw_norm_block
 CHUNK_QUANTUM = 4096
 ROW_SCALAR_BYTES = 64   # per table row, mi_adamw_step_capturable_rows
 
@@ -44,6 +45,7 @@ F_CLIP = 1 << 0
 F_BF16_COPY = 1 << 1
 F_WRITE_GRAD = 1 << 2
 F_AMSGRAD = 1 << 3
+F_NORM_BLOCK = 1 << 4
 
 T_VEC = 1 << 0
 
@@ -58,6 +60,8 @@ EXPORTS = (
     "mi_adamw_build_chunks",
     "mi_adamw_grad_norm",
     "mi_adamw_grad_norm_flat",
+    "mi_adamw_grad_norm_block",
+    "mi_adamw_grad_norm_block_flat",
     "mi_adamw_grad_norm_flat_noalloc",
     "mi_adamw_grad_sumsq",
     "mi_adamw_grad_sumsq_flat",
@@ -166,6 +170,8 @@ _SIGNATURES = {
     "mi_adamw_build_chunks": ([_vp, _i32, _i64, _vp, _i64], _i64),
     "mi_adamw_grad_norm": ([_vp, _vp, _i64, _i64, _f32, _vp, _vp, _vp, _vp], ctypes.c_int),
     "mi_adamw_grad_norm_flat": ([_vp, _i64, _i64, _f32, _vp, _vp, _vp, _vp], ctypes.c_int),
+    "mi_adamw_grad_norm_block": ([_vp, _vp, _i64, _i64, _f32, _f32, _vp, _vp, _vp], ctypes.c_int),
+    "mi_adamw_grad_norm_block_flat": ([_vp, _i64, _i64, _f32, _f32, _vp, _vp, _vp], ctypes.c_int),
     "mi_adamw_grad_norm_flat_noalloc": ([_vp, _i64, _i64, _f32, _vp, _vp, _vp], ctypes.c_int),
     "mi_adamw_grad_sumsq": ([_vp, _vp, _i64, _i64, _f32, _vp, _vp, _vp], ctypes.c_int),
     "mi_adamw_grad_sumsq_flat": ([_vp, _i64, _i64, _f32, _vp, _vp, _vp], ctypes.c_int),
@@ -197,9 +203,8 @@ _lib = None
 _host = None
 
 # The entry points the host extension calls, in the order _host.bind takes them.
-HOST_BINDINGS = ("mi_adamw_set_grads", "mi_adamw_grad_norm", "mi_adamw_grad_norm_flat",
-                 "mi_adamw_grad_sumsq", "mi_adamw_grad_sumsq_flat", "mi_adamw_norm_from_sumsq",
-                 "mi_adamw_step_prescaled", "mi_adamw_step_flat_prescaled",
+HOST_BINDINGS = ("mi_adamw_set_grads", "mi_adamw_grad_norm_block",
+                 "mi_adamw_grad_norm_block_flat", "mi_adamw_step_prescaled", "mi_adamw_step_flat_prescaled",
                  "mi_adamw_step_fused_chain", "mi_adamw_step_flat_fused_chain")
 
 

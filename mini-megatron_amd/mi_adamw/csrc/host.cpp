@@ -23,7 +23,7 @@
 //   plan(...) -> capsule                one launch's bookkeeping (see plan_new)
 //   prepare(plan, stream) -> int        steps 1-3: READY, READY_MOVED, FALLBACK or ERROR
 //   last_error(plan) -> int             the library's code behind the last ERROR
-//   norm(plan, stream, d_norm) -> int   mi_adamw_grad_norm* (or sumsq + finalize)
+//   norm(plan, stream, d_norm) -> int   mi_adamw_grad_norm_block*
 //   update(plan, stream, hypers, n) -> int   mi_adamw_step*_prescaled, or with the
 //                                       fused=True chain mi_adamw_step*_fused_chain
 //   sync_versions(plan, dict)           dict[id(p)] = (p._version, p.data_ptr())
@@ -55,15 +55,10 @@ constexpr int kError = 3;
 struct Api {
     int (*set_grads)(mi_adamw_tensor*, int32_t, int32_t, const int32_t*, const uint64_t*,
                      const uint8_t*, void*) = nullptr;
-    int (*grad_norm)(const mi_adamw_tensor*, const mi_adamw_chunk*, int64_t, int64_t, float,
-                     double*, float*, float*, void*) = nullptr;
-    int (*grad_norm_flat)(const float*, int64_t, int64_t, float, double*, float*, float*,
-                          void*) = nullptr;
-    int (*grad_sumsq)(const mi_adamw_tensor*, const mi_adamw_chunk*, int64_t, int64_t, float,
-                      double*, double*, void*) = nullptr;
-    int (*grad_sumsq_flat)(const float*, int64_t, int64_t, float, double*, double*,
-                           void*) = nullptr;
-    int (*norm_from_sumsq)(const double*, int32_t, float, float*, float*, void*) = nullptr;
+    int (*grad_norm_block)(const mi_adamw_tensor*, const mi_adamw_chunk*, int64_t, int64_t,
+                           float, float, mi_adamw_norm_block*, float*, void*) = nullptr;
+    int (*grad_norm_block_flat)(const float*, int64_t, int64_t, float, float,
+                                mi_adamw_norm_block*, float*, void*) = nullptr;
     int (*step_prescaled)(const mi_adamw_tensor*, const mi_adamw_chunk*, int64_t, int64_t,
                           const mi_adamw_hyper*, int32_t, const float*, float, int32_t, int32_t,
                           int32_t, void*) = nullptr;
@@ -120,9 +115,8 @@ struct Plan {
     bool clip = false;
     bool fused_chain = false;        // the hyperparameter sets are mi_adamw_fused_hyper
     float max_norm = 0.0f, prescale = 1.0f;
-    double* partials = nullptr;
-    float* coef = nullptr;
-    double* sumsq = nullptr;
+    mi_adamw_norm_block* block = nullptr;   // with clip: the norm pass's, read by the update
+    const float* scale = nullptr;           // what the update takes as its gradient scale
     uint64_t stream = 0;             // the stream the tables were last used on
     int last_error = 0;              // library code of prepare()'s last kError
     // scratch of prepare()
@@ -158,9 +152,9 @@ bool is_tensor(PyObject* obj) { return obj && THPVariable_Check(obj); }
 // ---------------------------------------------------------------------------
 
 PyObject* py_bind(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
-    constexpr int kN = 10;
+    constexpr int kN = 7;
     if (nargs != kN) {
-        PyErr_SetString(PyExc_TypeError, "bind: 10 function addresses");
+        PyErr_SetString(PyExc_TypeError, "bind: 7 function addresses");
         return nullptr;
     }
     void* a[kN];
@@ -172,15 +166,12 @@ PyObject* py_bind(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
         }
     }
     std::memcpy(&g_api.set_grads, &a[0], sizeof(void*));
-    std::memcpy(&g_api.grad_norm, &a[1], sizeof(void*));
-    std::memcpy(&g_api.grad_norm_flat, &a[2], sizeof(void*));
-    std::memcpy(&g_api.grad_sumsq, &a[3], sizeof(void*));
-    std::memcpy(&g_api.grad_sumsq_flat, &a[4], sizeof(void*));
-    std::memcpy(&g_api.norm_from_sumsq, &a[5], sizeof(void*));
-    std::memcpy(&g_api.step_prescaled, &a[6], sizeof(void*));
-    std::memcpy(&g_api.step_flat_prescaled, &a[7], sizeof(void*));
-    std::memcpy(&g_api.step_fused_chain, &a[8], sizeof(void*));
-    std::memcpy(&g_api.step_flat_fused_chain, &a[9], sizeof(void*));
+    std::memcpy(&g_api.grad_norm_block, &a[1], sizeof(void*));
+    std::memcpy(&g_api.grad_norm_block_flat, &a[2], sizeof(void*));
+    std::memcpy(&g_api.step_prescaled, &a[3], sizeof(void*));
+    std::memcpy(&g_api.step_flat_prescaled, &a[4], sizeof(void*));
+    std::memcpy(&g_api.step_fused_chain, &a[5], sizeof(void*));
+    std::memcpy(&g_api.step_flat_fused_chain, &a[6], sizeof(void*));
     g_bound = true;
     Py_RETURN_NONE;
 }
@@ -196,7 +187,7 @@ PyObject* py_bind(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
 //   launch:          (tables, d_rows, d_chunks, n_chunks, n_rows, host_rows, flat_row_addr,
 //                     flat_hyper)
 //   options:         (chunk_elems, max_blocks, state_code, flags, clip, max_norm, prescale,
-//                     partials, coef, sumsq, stream, fused_chain)
+//                     norm_block, grad_scale, 0, stream, fused_chain)
 //   keep:            objects to keep alive while the plan exists
 PyObject* plan_new(PyObject* args);
 
@@ -276,9 +267,9 @@ PyObject* plan_new(PyObject* args) {
         long long chunk = 0;
         int max_blocks = 0, state_code = 0, flags = 0, clip = 0, fused_chain = 0;
         float max_norm = 0, prescale = 1;
-        unsigned long long partials = 0, coef = 0, sumsq = 0, stream = 0;
+        unsigned long long block = 0, scale = 0, unused = 0, stream = 0;
         if (!PyArg_ParseTuple(opts_t, "LiiipffKKKKp", &chunk, &max_blocks, &state_code, &flags,
-                              &clip, &max_norm, &prescale, &partials, &coef, &sumsq, &stream,
+                              &clip, &max_norm, &prescale, &block, &scale, &unused, &stream,
                               &fused_chain))
             goto fail;
         pl->fused_chain = fused_chain;
@@ -289,9 +280,8 @@ PyObject* plan_new(PyObject* args) {
         pl->clip = clip;
         pl->max_norm = max_norm;
         pl->prescale = prescale;
-        pl->partials = reinterpret_cast<double*>(partials);
-        pl->coef = reinterpret_cast<float*>(coef);
-        pl->sumsq = reinterpret_cast<double*>(sumsq);
+        pl->block = reinterpret_cast<mi_adamw_norm_block*>(block);
+        pl->scale = reinterpret_cast<const float*>(scale);
         pl->stream = stream;
     }
     pl->e.resize(n);
@@ -483,23 +473,13 @@ PyObject* py_norm(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     void* s = PyLong_AsVoidPtr(args[1]);
     float* norm = static_cast<float*>(PyLong_AsVoidPtr(args[2]));
     if (PyErr_Occurred()) return nullptr;
-    int rc;
-    if (pl->prescale != 1.0f) {
-        rc = pl->tables ? g_api.grad_sumsq(pl->d_rows, pl->d_chunks, pl->n_chunks,
-                                           pl->chunk_elems, pl->prescale, pl->partials,
-                                           pl->sumsq, s)
-                        : g_api.grad_sumsq_flat(pl->flat_row.grad, pl->flat_row.numel,
-                                                pl->chunk_elems, pl->prescale, pl->partials,
-                                                pl->sumsq, s);
-        if (rc == MI_ADAMW_OK)
-            rc = g_api.norm_from_sumsq(pl->sumsq, 1, pl->max_norm, norm, pl->coef, s);
-    } else {
-        rc = pl->tables ? g_api.grad_norm(pl->d_rows, pl->d_chunks, pl->n_chunks, pl->chunk_elems,
-                                          pl->max_norm, pl->partials, norm, pl->coef, s)
-                        : g_api.grad_norm_flat(pl->flat_row.grad, pl->flat_row.numel,
-                                               pl->chunk_elems, pl->max_norm, pl->partials, norm,
-                                               pl->coef, s);
-    }
+    const int rc =
+        pl->tables ? g_api.grad_norm_block(pl->d_rows, pl->d_chunks, pl->n_chunks,
+                                           pl->chunk_elems, pl->prescale, pl->max_norm,
+                                           pl->block, norm, s)
+                   : g_api.grad_norm_block_flat(pl->flat_row.grad, pl->flat_row.numel,
+                                                pl->chunk_elems, pl->prescale, pl->max_norm,
+                                                pl->block, norm, s);
     return PyLong_FromLong(rc);
 }
 
@@ -514,18 +494,18 @@ PyObject* py_update(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     void* hv = PyLong_AsVoidPtr(args[2]);
     const long nh = PyLong_AsLong(args[3]);
     if (PyErr_Occurred()) return nullptr;
-    const int32_t flags = pl->flags | (pl->clip ? MI_ADAMW_F_CLIP : 0);
+    const int32_t flags = pl->flags | (pl->clip ? MI_ADAMW_F_CLIP | MI_ADAMW_F_NORM_BLOCK : 0);
     int rc;
     if (pl->fused_chain) {
         const mi_adamw_fused_hyper* fh = static_cast<const mi_adamw_fused_hyper*>(hv);
         if (pl->tables) {
             rc = g_api.step_fused_chain(pl->d_rows, pl->d_chunks, pl->n_chunks, pl->chunk_elems,
                                         fh, static_cast<int32_t>(nh), nullptr, nullptr,
-                                        pl->coef, pl->prescale, pl->state_code, flags,
+                                        pl->scale, pl->prescale, pl->state_code, flags,
                                         pl->max_blocks, s);
         } else {
             if (pl->flat_hyper >= nh) return PyLong_FromLong(MI_ADAMW_E_INVALID);
-            rc = g_api.step_flat_fused_chain(&pl->flat_row, fh + pl->flat_hyper, pl->coef,
+            rc = g_api.step_flat_fused_chain(&pl->flat_row, fh + pl->flat_hyper, pl->scale,
                                              pl->prescale, pl->chunk_elems, pl->state_code,
                                              flags, pl->max_blocks, s);
         }
@@ -534,11 +514,11 @@ PyObject* py_update(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     const mi_adamw_hyper* h = static_cast<const mi_adamw_hyper*>(hv);
     if (pl->tables) {
         rc = g_api.step_prescaled(pl->d_rows, pl->d_chunks, pl->n_chunks, pl->chunk_elems, h,
-                                  static_cast<int32_t>(nh), pl->coef, pl->prescale,
+                                  static_cast<int32_t>(nh), pl->scale, pl->prescale,
                                   pl->state_code, flags, pl->max_blocks, s);
     } else {
         if (pl->flat_hyper >= nh) return PyLong_FromLong(MI_ADAMW_E_INVALID);
-        rc = g_api.step_flat_prescaled(&pl->flat_row, h + pl->flat_hyper, pl->coef, pl->prescale,
+        rc = g_api.step_flat_prescaled(&pl->flat_row, h + pl->flat_hyper, pl->scale, pl->prescale,
                                        pl->chunk_elems, pl->state_code, flags, pl->max_blocks, s);
     }
     return PyLong_FromLong(rc);

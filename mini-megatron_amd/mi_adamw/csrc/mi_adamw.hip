@@ -76,6 +76,9 @@ static_assert(offsetof(mi_adamw_tensor, max_exp_avg_sq) == 40 &&
               offsetof(mi_adamw_tensor, numel) == 48, "pointer words, then numel");
 static_assert(offsetof(mi_adamw_tensor, hyper) == 56 && offsetof(mi_adamw_tensor, flags) == 60,
               "hyper and flags share the last word");
+static_assert(sizeof(mi_adamw_norm_block) == MI_ADAMW_NORM_BLOCK_BYTES &&
+                  offsetof(mi_adamw_norm_block, norm) == 4096,
+              "mi_adamw_norm_block: the partial sums, then one 64-byte line");
 static_assert(sizeof(mi_adamw_chunk) == 8, "mi_adamw_chunk is two int32");
 static_assert(sizeof(mi_adamw_capt_hyper) == 48 && offsetof(mi_adamw_capt_hyper, lr_ptr) == 40,
               "mi_adamw_capt_hyper: ten 4-byte fields, then the lr pointer");
@@ -742,10 +745,20 @@ struct ReverseSource {
 // 0.2-0.6% off the update against keeping the chunks the update reads last, which its own
 // traffic evicts first).  Two loops, not one with a per-chunk choice: the compiler would
 // fold the two loads into one.
+//
+// Block: the clip's device memory (null outside mi_adamw_grad_norm_block*), which the
+// update reads; workgroup 0 writes its fields.
+struct BlockArgs {
+    mi_adamw_norm_block* block;
+    float* norm;
+    float max_norm;
+    int32_t n_partials;
+};
+
 template <class Src>
 __global__ __launch_bounds__(kNormThreads) void mi_adamw_sumsq_kernel(
     Src src, int64_t n_chunks, int64_t chunk_elems, double* __restrict__ partials,
-    int64_t keep_from, float pre) {
+    int64_t keep_from, float pre, BlockArgs ba) {
     double acc0 = 0.0, acc1 = 0.0;
     int64_t c = blockIdx.x;
     const ReverseSource<Src> rev{src, n_chunks};
@@ -753,26 +766,61 @@ __global__ __launch_bounds__(kNormThreads) void mi_adamw_sumsq_kernel(
     sumsq_chunks<true>(rev, c, n_chunks, gridDim.x, chunk_elems, pre, acc0, acc1);
     const double total = block_sum<kNormThreads>(acc0 + acc1);
     if (threadIdx.x == 0) partials[blockIdx.x] = total;
+    if (ba.block && blockIdx.x == 0 && threadIdx.x == 0) {
+        ba.block->norm = ba.norm;
+        ba.block->max_norm = ba.max_norm;
+        ba.block->n_partials = ba.n_partials;
+    }
 }
 
-// One workgroup: reduce the partial sums in a fixed order, then the norm and
-// the clip coefficient.  Running as its own launch, it sees every partial
-// through the kernel boundary; no fence or completion counter is needed.
+// The partial sums in a fixed order by the first kNormThreads threads of a workgroup of
+// kThreads (the others add zeros); the sum is valid in thread 0.
+template <int kThreads>
+__device__ __forceinline__ double sum_partials(const double* __restrict__ partials,
+                                               int n_partials) {
+    double s = 0.0;
+    if (threadIdx.x < kNormThreads)
+        for (int i = threadIdx.x; i < n_partials; i += kNormThreads) s += partials[i];
+    return block_sum<kThreads>(s);
+}
+
+// clip_grad.py:165-169: t = norm + 1e-6; coef = max_norm * (1/t); clamp(max=1)
+__device__ __forceinline__ float clip_coef(float norm, float max_norm) {
+    const float tt = norm + 1e-6f;
+    const float r = 1.0f / tt;
+    const float coef = r * max_norm;
+    return coef > 1.0f ? 1.0f : coef;  // NaN stays NaN, as torch.clamp
+}
+
+// One workgroup: reduce the partial sums, then the norm and the clip coefficient.  Running
+// as its own launch, it sees every partial through the kernel boundary; no fence or
+// completion counter is needed.
 __global__ __launch_bounds__(kNormThreads) void mi_adamw_norm_finalize_kernel(
     const double* __restrict__ partials, int n_partials, float max_norm,
     float* __restrict__ norm_out, float* __restrict__ coef_out) {
-    double s = 0.0;
-    for (int i = threadIdx.x; i < n_partials; i += kNormThreads) s += partials[i];
-    s = block_sum<kNormThreads>(s);
+    const double s = sum_partials<kNormThreads>(partials, n_partials);
     if (threadIdx.x == 0) {
         const float norm = static_cast<float>(__builtin_sqrt(s));
-        // clip_grad.py:165-169: t = norm + 1e-6; coef = max_norm * (1/t); clamp(max=1)
-        const float tt = norm + 1e-6f;
-        const float r = 1.0f / tt;
-        const float coef = r * max_norm;
         *norm_out = norm;
-        *coef_out = coef > 1.0f ? 1.0f : coef;  // NaN stays NaN, as torch.clamp
+        *coef_out = clip_coef(norm, max_norm);
     }
+}
+
+// The same in every workgroup of the launch that needs the coefficient (the update with
+// MI_ADAMW_F_NORM_BLOCK): called by all its threads, once its first tile's loads are in
+// flight, whose latency covers most of it; workgroup 0 writes the norm out.  It saves a
+// launch where few workgroups pay for it (kFoldElems).
+template <int kThreads>
+__device__ __forceinline__ float block_coef(const mi_adamw_norm_block* b, int32_t n) {
+    __shared__ float coef;
+    const double s = sum_partials<kThreads>(b->partials, n);
+    if (threadIdx.x == 0) {
+        const float norm = static_cast<float>(__builtin_sqrt(s));
+        coef = clip_coef(norm, *(const CONSTANT float*)(&b->max_norm));
+        if (blockIdx.x == 0) **(float* const CONSTANT*)(&b->norm) = norm;
+    }
+    __syncthreads();
+    return __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(coef)));
 }
 
 // One workgroup: the partial sums of one range reduced to its float64 sum of squares,
@@ -781,9 +829,7 @@ __global__ __launch_bounds__(kNormThreads) void mi_adamw_norm_finalize_kernel(
 // the partials themselves (0 + s == s, and s + 0 == s for s >= 0).
 __global__ __launch_bounds__(kNormThreads) void mi_adamw_sumsq_reduce_kernel(
     const double* __restrict__ partials, int n_partials, double* __restrict__ sumsq_out) {
-    double s = 0.0;
-    for (int i = threadIdx.x; i < n_partials; i += kNormThreads) s += partials[i];
-    s = block_sum<kNormThreads>(s);
+    const double s = sum_partials<kNormThreads>(partials, n_partials);
     if (threadIdx.x == 0) *sumsq_out = s;
 }
 
@@ -900,7 +946,11 @@ __device__ __forceinline__ typename HS::Scalars shared_scalars(const HS& hs,
     return r;
 }
 
-template <class Src, class HS, typename StateT, bool kClip, bool kCopy, bool kWriteGrad, bool kAms>
+// Where the clip coefficient comes from: no clip, a float in device memory, or a
+// mi_adamw_norm_block (block_coef).
+enum Clip { kNoClip, kCoef, kBlock };
+
+template <class Src, class HS, typename StateT, Clip kClip, bool kCopy, bool kWriteGrad, bool kAms>
 __global__ __launch_bounds__(update_threads<HS>())
 __attribute__((amdgpu_waves_per_eu(4, 4)))   // the cap above, and 128 VGPRs per lane
 void mi_adamw_update_kernel(
@@ -912,7 +962,14 @@ void mi_adamw_update_kernel(
     constexpr bool kCapt = HS::kCapt;
     constexpr bool kLate = HS::kLate;
     constexpr bool kProbe = HS::kProbe;
-    const float scale = kClip ? *grad_scale : 1.0f;
+    float scale = kClip == kCoef ? *grad_scale : 1.0f;
+    int32_t n_partials = 0;         // kBlock: partial sums still to be reduced
+    if (kClip == kBlock) {
+        // written by the launch before this one, unchanged during it: scalar loads
+        const mi_adamw_norm_block* b = reinterpret_cast<const mi_adamw_norm_block*>(grad_scale);
+        n_partials = *(const CONSTANT int32_t*)(&b->n_partials);
+        scale = *(const CONSTANT float*)(&b->coef);
+    }
     int parity = 0;   // shared_scalars' buffer of this item
     for (int64_t w = blockIdx.x; w < items.n; w += gridDim.x) {
         mi_adamw_tensor t;
@@ -946,11 +1003,17 @@ void mi_adamw_update_kernel(
                 h = hs.get(t, row);
             }
         }
+        if (kClip == kBlock && n_partials) {
+            __builtin_amdgcn_sched_barrier(0);
+            scale = block_coef<kThreads>(reinterpret_cast<const mi_adamw_norm_block*>(grad_scale),
+                                         n_partials);
+            n_partials = 0;
+        }
         const float gmul = h.grad_sign;
         if (have) {
             // the stored value of div_(world), then of the clip, then -g with maximize
             f32x4 gs = f32x4{cur.g.x * pre, cur.g.y * pre, cur.g.z * pre, cur.g.w * pre};
-            if (kClip) gs = f32x4{gs.x * scale, gs.y * scale, gs.z * scale, gs.w * scale};
+            if (kClip != kNoClip) gs = f32x4{gs.x * scale, gs.y * scale, gs.z * scale, gs.w * scale};
             if (kWriteGrad) st4(G + i, gs);
             if (kProbe) {
                 keep(gs);
@@ -967,7 +1030,7 @@ void mi_adamw_update_kernel(
         // the tensor's last elements, up to three
         for (int64_t j = vend + threadIdx.x; j < end; j += kThreads) {
             float g1 = ld1(G + j) * pre;
-            if (kClip) g1 = g1 * scale;
+            if (kClip != kNoClip) g1 = g1 * scale;
             if (kWriteGrad) st1(G + j, g1);
             g1 = g1 * gmul;
             float p1 = ld1(P + j), m1 = IO::ld1(M, j), v1 = IO::ld1(V, j);
@@ -1082,6 +1145,12 @@ constexpr int kNormBlocks = 512;
 #endif
 constexpr int64_t kNormKeepBytes = int64_t(MI_ADAMW_NORM_KEEP_MB) << 20;
 
+// Largest set whose update reduces the partial sums itself: 1024 of its workgroups are
+// resident at once, so up to here each of the chip's slots does so once.  0.1M parameters,
+// clip, 24.5 us with the finalize launch, 21.5 without; 5.4M (five rounds of workgroups) 46.5
+// against 52, 17M 90 against 101.
+constexpr int64_t kFoldElems = int64_t(1) << 20;
+
 bool chunk_elems_ok(int64_t chunk_elems) {
     return chunk_elems > 0 && (chunk_elems % kChunkQuantum) == 0 &&
            chunk_elems <= (int64_t(1) << 30);
@@ -1115,14 +1184,15 @@ bool finite(float x) { return x - x == 0.0f; }
 // (partials_cap doubles available).  Sets *grid_out to the number of partials written.
 template <class Src>
 int launch_sumsq(const Src& src, int64_t n_chunks, int64_t chunk_elems, float pre,
-                 double* partials, int64_t partials_cap, unsigned* grid_out, hipStream_t s) {
+                 double* partials, int64_t partials_cap, unsigned* grid_out, hipStream_t s,
+                 BlockArgs ba = BlockArgs{}) {
     if (n_chunks <= 0 || !chunk_elems_ok(chunk_elems) || !partials) return MI_ADAMW_E_INVALID;
     const unsigned grid = grid_for(n_chunks, kNormBlocks, kNormThreads);
     if (grid > partials_cap) return MI_ADAMW_E_SCRATCH;
     const int64_t keep_chunks = kNormKeepBytes / (chunk_elems * static_cast<int64_t>(sizeof(float)));
     const int64_t keep_from = n_chunks > keep_chunks ? n_chunks - keep_chunks : 0;
     hipLaunchKernelGGL(mi_adamw_sumsq_kernel<Src>, dim3(grid), dim3(kNormThreads), 0, s, src,
-                       n_chunks, chunk_elems, partials, keep_from, pre);
+                       n_chunks, chunk_elems, partials, keep_from, pre, ba);
     *grid_out = grid;
     return launch_status();
 }
@@ -1141,6 +1211,24 @@ int launch_norm(const Src& src, int64_t n_chunks, int64_t chunk_elems, float max
     return launch_status();
 }
 
+// Pass 1 into a norm block, the rest left to the update or, for a large set, finalized here.
+template <class Src>
+int launch_norm_block(const Src& src, int64_t n_chunks, int64_t chunk_elems, float pre,
+                      float max_norm, mi_adamw_norm_block* block, float* norm, hipStream_t s) {
+    if (!block || !norm || !aligned(block, 8) || !finite(pre)) return MI_ADAMW_E_INVALID;
+    if (n_chunks <= 0 || !chunk_elems_ok(chunk_elems)) return MI_ADAMW_E_INVALID;
+    const bool fold = n_chunks <= kFoldElems / chunk_elems;
+    const unsigned n = grid_for(n_chunks, kNormBlocks, kNormThreads);
+    const BlockArgs ba{block, norm, max_norm, fold ? static_cast<int32_t>(n) : 0};
+    unsigned grid = 0;
+    const int rc = launch_sumsq(src, n_chunks, chunk_elems, pre, block->partials,
+                                MI_ADAMW_NORM_BLOCK_PARTIALS, &grid, s, ba);
+    if (rc != MI_ADAMW_OK || fold) return rc;
+    hipLaunchKernelGGL(mi_adamw_norm_finalize_kernel, dim3(1), dim3(kNormThreads), 0, s,
+                       block->partials, static_cast<int>(grid), max_norm, norm, &block->coef);
+    return launch_status();
+}
+
 // Pass 1 and the reduction of its partials to one float64 sum of squares.
 template <class Src>
 int launch_sumsq_total(const Src& src, int64_t n_chunks, int64_t chunk_elems, float pre,
@@ -1155,7 +1243,7 @@ int launch_sumsq_total(const Src& src, int64_t n_chunks, int64_t chunk_elems, fl
     return launch_status();
 }
 
-template <class Src, class HS, typename StateT, bool kClip, bool kCopy, bool kWriteGrad,
+template <class Src, class HS, typename StateT, Clip kClip, bool kCopy, bool kWriteGrad,
           bool kAms>
 int launch_update_k(const Src& src, int64_t n_chunks, int64_t chunk_elems, const HS& hs,
                     const float* scale, float pre, int32_t max_blocks, hipStream_t s) {
@@ -1168,7 +1256,7 @@ int launch_update_k(const Src& src, int64_t n_chunks, int64_t chunk_elems, const
 }
 
 // Runtime flags -> kernel template: one instantiation per (copy, write-grad, amsgrad).
-template <class Src, class HS, typename StateT, bool kClip>
+template <class Src, class HS, typename StateT, Clip kClip>
 int launch_update_cw(const Src& src, int64_t n_chunks, int64_t chunk_elems, const HS& hs,
                      const float* scale, float pre, int32_t flags, int32_t max_blocks,
                      hipStream_t s) {
@@ -1201,19 +1289,20 @@ int launch_update(const Src& src, int64_t n_chunks, int64_t chunk_elems, const H
     if (state_dtype != MI_ADAMW_STATE_F32 && state_dtype != MI_ADAMW_STATE_BF16)
         return MI_ADAMW_E_INVALID;
     if (flags & ~(MI_ADAMW_F_CLIP | MI_ADAMW_F_BF16_COPY | MI_ADAMW_F_WRITE_GRAD |
-                  MI_ADAMW_F_AMSGRAD))
+                  MI_ADAMW_F_AMSGRAD | MI_ADAMW_F_NORM_BLOCK))
         return MI_ADAMW_E_INVALID;
-    const bool clip = flags & MI_ADAMW_F_CLIP;
-    if (clip && !scale) return MI_ADAMW_E_INVALID;
-    if (state_dtype == MI_ADAMW_STATE_F32)
-        return clip ? launch_update_cw<Src, HS, float, true>(src, n_chunks, chunk_elems, hs,
-                                                              scale, pre, flags, max_blocks, s)
-                    : launch_update_cw<Src, HS, float, false>(src, n_chunks, chunk_elems, hs,
-                                                               scale, pre, flags, max_blocks, s);
-    return clip ? launch_update_cw<Src, HS, uint16_t, true>(src, n_chunks, chunk_elems, hs, scale,
-                                                             pre, flags, max_blocks, s)
-                : launch_update_cw<Src, HS, uint16_t, false>(src, n_chunks, chunk_elems, hs,
-                                                              scale, pre, flags, max_blocks, s);
+    const bool clip = flags & MI_ADAMW_F_CLIP, block = flags & MI_ADAMW_F_NORM_BLOCK;
+    if (clip ? !scale : block) return MI_ADAMW_E_INVALID;
+    if (block && !aligned(scale, 8)) return MI_ADAMW_E_INVALID;
+#define MI_ADAMW_CLIP(S)                                                                       \
+    (block  ? launch_update_cw<Src, HS, S, kBlock>(src, n_chunks, chunk_elems, hs, scale, pre, \
+                                                   flags, max_blocks, s)                       \
+     : clip ? launch_update_cw<Src, HS, S, kCoef>(src, n_chunks, chunk_elems, hs, scale, pre,  \
+                                                  flags, max_blocks, s)                        \
+            : launch_update_cw<Src, HS, S, kNoClip>(src, n_chunks, chunk_elems, hs, scale,     \
+                                                    pre, flags, max_blocks, s))
+    return state_dtype == MI_ADAMW_STATE_F32 ? MI_ADAMW_CLIP(float) : MI_ADAMW_CLIP(uint16_t);
+#undef MI_ADAMW_CLIP
 }
 
 // The memory-only twin of launch_update (no clip: the gradient is read either way).
@@ -1228,9 +1317,9 @@ int launch_probe(const Src& src, int64_t n_chunks, int64_t chunk_elems, int32_t 
         return MI_ADAMW_E_INVALID;
     const ProbeHyper hs;
     if (state_dtype == MI_ADAMW_STATE_F32)
-        return launch_update_cw<Src, ProbeHyper, float, false>(src, n_chunks, chunk_elems, hs,
+        return launch_update_cw<Src, ProbeHyper, float, kNoClip>(src, n_chunks, chunk_elems, hs,
                                                                nullptr, 1.0f, flags, max_blocks, s);
-    return launch_update_cw<Src, ProbeHyper, uint16_t, false>(src, n_chunks, chunk_elems, hs,
+    return launch_update_cw<Src, ProbeHyper, uint16_t, kNoClip>(src, n_chunks, chunk_elems, hs,
                                                               nullptr, 1.0f, flags, max_blocks, s);
 }
 
@@ -1411,6 +1500,29 @@ int mi_adamw_grad_norm_flat(const float* d_grad, int64_t n, int64_t chunk_elems,
     const int64_t n_chunks = (n + chunk_elems - 1) / chunk_elems;
     return launch_norm(src, n_chunks, chunk_elems, max_norm, d_partials, d_norm, d_coef,
                        static_cast<hipStream_t>(stream));
+}
+
+int mi_adamw_grad_norm_block(const mi_adamw_tensor* d_tensors, const mi_adamw_chunk* d_chunks,
+                             int64_t n_chunks, int64_t chunk_elems, float grad_prescale,
+                             float max_norm, mi_adamw_norm_block* d_block, float* d_norm,
+                             void* stream) {
+    if (!d_tensors || !d_chunks) return MI_ADAMW_E_INVALID;
+    TableSource src{d_tensors, d_chunks};
+    return launch_norm_block(src, n_chunks, chunk_elems, grad_prescale, max_norm, d_block, d_norm,
+                             static_cast<hipStream_t>(stream));
+}
+
+int mi_adamw_grad_norm_block_flat(const float* d_grad, int64_t n, int64_t chunk_elems,
+                                  float grad_prescale, float max_norm,
+                                  mi_adamw_norm_block* d_block, float* d_norm, void* stream) {
+    if (!d_grad || n <= 0 || !chunk_elems_ok(chunk_elems)) return MI_ADAMW_E_INVALID;
+    FlatSource src;
+    memset(&src.t, 0, sizeof(src.t));
+    src.t.grad = const_cast<float*>(d_grad);
+    src.t.numel = n;
+    const int64_t n_chunks = (n + chunk_elems - 1) / chunk_elems;
+    return launch_norm_block(src, n_chunks, chunk_elems, grad_prescale, max_norm, d_block, d_norm,
+                             static_cast<hipStream_t>(stream));
 }
 
 int mi_adamw_grad_norm_flat_noalloc(const float* d_grad, int64_t n, int64_t chunk_elems,

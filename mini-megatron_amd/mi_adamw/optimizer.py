@@ -968,7 +968,7 @@ class FusedAdamW(Optimizer):
                      for g in self.param_groups)
 
     def _make_fast(self, entries, hyper_idx, hyper_group, ams, fused, launch, device, stream,
-                   partials, coef, state_code, flags):
+                   block, state_code, flags):
         """The native path's plan for the steps after this one, when this step's launch is
         one the native path can repeat: every parameter stepped, one launch that the norm
         pass shares, one hyperparameter set per param group."""
@@ -990,7 +990,6 @@ class FusedAdamW(Optimizer):
         flat_row = None if launch.tables else self._row_struct(launch)
         if ams:
             flags |= _lib.F_AMSGRAD
-        sumsq = self._sumsq_buf(device) if self.grad_prescale != 1.0 else None
         clip = self.max_grad_norm is not None
         if not clip:
             flags &= ~_lib.F_WRITE_GRAD
@@ -1008,10 +1007,9 @@ class FusedAdamW(Optimizer):
                  0 if launch.tables else int(launch.host_rows[0]["hyper"])),
                 (int(self.chunk_elems), int(self.max_blocks), int(state_code), int(flags), clip,
                  float(self.max_grad_norm or 0.0), float(self.grad_prescale),
-                 partials.data_ptr(), coef.data_ptr(), 0 if sumsq is None else sumsq.data_ptr(),
-                 int(stream), bool(fused)),
+                 block.data_ptr(), block.data_ptr(), 0, int(stream), bool(fused)),
                 (launch.rows, launch.chunks, launch.host_rows, self._steps, hyper_steps,
-                 partials, coef, sumsq))
+                 block))
         except (TypeError, ValueError):
             return None     # a state entry the plan cannot check (not a tensor): general path
         fast = _Fast()
@@ -1101,12 +1099,13 @@ class FusedAdamW(Optimizer):
             ws = self._workspace[device] = (partials, coef)
         return ws
 
-    def _sumsq_buf(self, device: torch.device) -> torch.Tensor:
-        """One float64 on the device: the pre-scaled gradients' sum of squares."""
-        buf = self._workspace.get(("sumsq", device))
+    def _norm_block(self, device: torch.device) -> torch.Tensor:
+        """The device memory that carries a step's clip from its norm pass to its update
+        (mi_adamw_norm_block)."""
+        buf = self._workspace.get(("norm block", device))
         if buf is None:
-            buf = self._workspace[("sumsq", device)] = torch.zeros(1, dtype=torch.float64,
-                                                                    device=device)
+            buf = self._workspace[("norm block", device)] = torch.zeros(
+                _lib.NORM_BLOCK_BYTES, dtype=torch.uint8, device=device)
         return buf
 
     def _rows(self, entries, hyper_idx, ams):
@@ -1229,7 +1228,7 @@ class FusedAdamW(Optimizer):
         lib = _lib.load()
         self._fast = None
         stream = torch.cuda.current_stream(device).cuda_stream
-        partials, coef = self._ws(device)
+        norm_block = self._norm_block(device)
         flags = 0
         if self.bf16_copy:
             flags |= _lib.F_BF16_COPY
@@ -1295,37 +1294,20 @@ class FusedAdamW(Optimizer):
             if norm_launch.n_chunks == 0:
                 # nothing but empty tensors: torch's norm of no elements is 0
                 norm.zero_()
-                coef.fill_(1.0)
-            elif self.grad_prescale != 1.0:
-                # the sum of squares of the pre-scaled gradients, then the finalize over it
-                sumsq = self._sumsq_buf(device)
-                if norm_launch.n_rows == 1:
-                    row = self._row_struct(norm_launch)
-                    _lib.check(lib.mi_adamw_grad_sumsq_flat(
-                        row.grad, row.numel, self.chunk_elems, self.grad_prescale,
-                        partials.data_ptr(), sumsq.data_ptr(), stream), "mi_adamw_grad_sumsq_flat")
-                else:
-                    _lib.check(lib.mi_adamw_grad_sumsq(
-                        norm_launch.rows.data_ptr(), norm_launch.chunks.data_ptr(),
-                        norm_launch.n_chunks, self.chunk_elems, self.grad_prescale,
-                        partials.data_ptr(), sumsq.data_ptr(), stream), "mi_adamw_grad_sumsq")
-                _lib.check(lib.mi_adamw_norm_from_sumsq(
-                    sumsq.data_ptr(), 1, float(self.max_grad_norm), norm.data_ptr(),
-                    coef.data_ptr(), stream), "mi_adamw_norm_from_sumsq")
             elif norm_launch.n_rows == 1:
                 row = self._row_struct(norm_launch)
-                _lib.check(lib.mi_adamw_grad_norm_flat(
-                    row.grad, row.numel, self.chunk_elems, float(self.max_grad_norm),
-                    partials.data_ptr(), norm.data_ptr(), coef.data_ptr(),
-                    stream), "mi_adamw_grad_norm_flat")
+                _lib.check(lib.mi_adamw_grad_norm_block_flat(
+                    row.grad, row.numel, self.chunk_elems, self.grad_prescale,
+                    float(self.max_grad_norm), norm_block.data_ptr(), norm.data_ptr(), stream),
+                    "mi_adamw_grad_norm_block_flat")
             else:
-                _lib.check(lib.mi_adamw_grad_norm(
+                _lib.check(lib.mi_adamw_grad_norm_block(
                     norm_launch.rows.data_ptr(), norm_launch.chunks.data_ptr(),
-                    norm_launch.n_chunks, self.chunk_elems, float(self.max_grad_norm),
-                    partials.data_ptr(), norm.data_ptr(), coef.data_ptr(),
-                    stream), "mi_adamw_grad_norm")
+                    norm_launch.n_chunks, self.chunk_elems, self.grad_prescale,
+                    float(self.max_grad_norm), norm_block.data_ptr(), norm.data_ptr(), stream),
+                    "mi_adamw_grad_norm_block")
             self.last_grad_norm = norm
-            flags |= _lib.F_CLIP
+            flags |= _lib.F_CLIP | _lib.F_NORM_BLOCK
             if self.clip_write_grads:
                 flags |= _lib.F_WRITE_GRAD
         _record(ev, 1)
@@ -1334,7 +1316,7 @@ class FusedAdamW(Optimizer):
                 continue
             lflags = flags | (_lib.F_AMSGRAD if ams else 0)
             if fused:
-                self._launch_fused_chain(launch, hs, coef, state_code, lflags, stream)
+                self._launch_fused_chain(launch, hs, norm_block, state_code, lflags, stream)
                 continue
             if self.capturable:
                 carr = (_lib.CaptHyper * len(hs))(*hs)
@@ -1342,7 +1324,7 @@ class FusedAdamW(Optimizer):
                     launch.rows.data_ptr(), launch.n_rows, launch.chunks.data_ptr(),
                     launch.n_chunks, self.chunk_elems, carr, len(hs), self._steps.data_ptr(),
                     launch.step_index.data_ptr(), launch.row_scalars.data_ptr(),
-                    coef.data_ptr(), state_code, lflags, self.max_blocks, stream),
+                    norm_block.data_ptr(), state_code, lflags, self.max_blocks, stream),
                     "mi_adamw_step_capturable_rows")
                 continue
             harr = (_lib.Hyper * len(hs))(*hs)
@@ -1352,31 +1334,32 @@ class FusedAdamW(Optimizer):
                 row_h = hs[int(launch.host_rows[0]["hyper"])]
                 if pre != 1.0:
                     _lib.check(lib.mi_adamw_step_flat_prescaled(
-                        ctypes.byref(row), ctypes.byref(row_h), coef.data_ptr(), pre,
+                        ctypes.byref(row), ctypes.byref(row_h), norm_block.data_ptr(), pre,
                         self.chunk_elems, state_code, lflags, self.max_blocks, stream),
                         "mi_adamw_step_flat_prescaled")
                     continue
                 _lib.check(lib.mi_adamw_step_flat(
-                    ctypes.byref(row), ctypes.byref(row_h), coef.data_ptr(), self.chunk_elems,
+                    ctypes.byref(row), ctypes.byref(row_h), norm_block.data_ptr(), self.chunk_elems,
                     state_code, lflags, self.max_blocks, stream), "mi_adamw_step_flat")
                 continue
             if pre != 1.0:
                 _lib.check(lib.mi_adamw_step_prescaled(
                     launch.rows.data_ptr(), launch.chunks.data_ptr(), launch.n_chunks,
-                    self.chunk_elems, harr, len(hs), coef.data_ptr(), pre, state_code, lflags,
+                    self.chunk_elems, harr, len(hs), norm_block.data_ptr(), pre, state_code, lflags,
                     self.max_blocks, stream), "mi_adamw_step_prescaled")
                 continue
             _lib.check(lib.mi_adamw_step(
                 launch.rows.data_ptr(), launch.chunks.data_ptr(), launch.n_chunks,
-                self.chunk_elems, harr, len(hs), coef.data_ptr(), state_code, lflags,
+                self.chunk_elems, harr, len(hs), norm_block.data_ptr(), state_code, lflags,
                 self.max_blocks, stream), "mi_adamw_step")
         _record(ev, 2)
         if len(parts) == 1 and hyper_group is not None:
             self._fast = self._make_fast(entries, hyper_idx, hyper_group, hyper_ams[0],
-                                         hyper_fused[0], launches[0], device, stream, partials,
-                                         coef, state_code, flags & ~_lib.F_CLIP)
+                                         hyper_fused[0], launches[0], device, stream, norm_block,
+                                         state_code,
+                                         flags & ~(_lib.F_CLIP | _lib.F_NORM_BLOCK))
 
-    def _launch_fused_chain(self, launch: _Launch, hs: list, coef: torch.Tensor,
+    def _launch_fused_chain(self, launch: _Launch, hs: list, block: torch.Tensor,
                             state_code: int, flags: int, stream: int) -> None:
         """One launch of torch's fused=True chain: the tables (with the device step counts
         when capturable) or the one flat range."""
@@ -1386,7 +1369,7 @@ class FusedAdamW(Optimizer):
             row = self._row_struct(launch)
             row_h = hs[int(launch.host_rows[0]["hyper"])]
             _lib.check(lib.mi_adamw_step_flat_fused_chain(
-                ctypes.byref(row), ctypes.byref(row_h), coef.data_ptr(), pre, self.chunk_elems,
+                ctypes.byref(row), ctypes.byref(row_h), block.data_ptr(), pre, self.chunk_elems,
                 state_code, flags, self.max_blocks, stream), "mi_adamw_step_flat_fused_chain")
             return
         farr = (_lib.FusedHyper * len(hs))(*hs)
@@ -1395,12 +1378,12 @@ class FusedAdamW(Optimizer):
             _lib.check(lib.mi_adamw_step_fused_chain_rows(
                 launch.rows.data_ptr(), launch.n_rows, launch.chunks.data_ptr(), launch.n_chunks,
                 self.chunk_elems, farr, len(hs), self._steps.data_ptr(),
-                launch.step_index.data_ptr(), launch.row_scalars.data_ptr(), coef.data_ptr(),
+                launch.step_index.data_ptr(), launch.row_scalars.data_ptr(), block.data_ptr(),
                 pre, state_code, flags, self.max_blocks, stream),
                 "mi_adamw_step_fused_chain_rows")
             return
         # host step counts (hs[i].step): no step buffer
         _lib.check(lib.mi_adamw_step_fused_chain(
             launch.rows.data_ptr(), launch.chunks.data_ptr(), launch.n_chunks, self.chunk_elems,
-            farr, len(hs), None, None, coef.data_ptr(), pre, state_code, flags, self.max_blocks,
+            farr, len(hs), None, None, block.data_ptr(), pre, state_code, flags, self.max_blocks,
             stream), "mi_adamw_step_fused_chain")
