@@ -68,6 +68,12 @@ extern "C" {
                                           mi_adamw_norm_block (cast to const float *) that
                                           mi_adamw_grad_norm_block* wrote earlier on the stream */
 
+#define MI_ADAMW_F_ADVANCE (1 << 5)    /* mi_adamw_step_capturable_rows and _fused_chain_rows:
+                                          d_steps holds the counts before this step; the launch
+                                          that forms the rows' values adds 1 to each row's count
+                                          first (every row then has an index of its own), in
+                                          place of a launch that increments them (adam.py:414) */
+
 /* mi_adamw_tensor.flags */
 #define MI_ADAMW_T_VEC (1 << 0) /* promises fp32 pointers 16-byte aligned and bf16 pointers
                                    8-byte aligned (the flat entry points check it); the
@@ -217,11 +223,13 @@ typedef struct mi_adamw_norm_block {
  * by the update launched next on the stream with MI_ADAMW_F_CLIP | MI_ADAMW_F_NORM_BLOCK and
  * d_grad_scale = (const float *)d_block.  *d_norm is written by then.  Sets too large to
  * gain from that (every workgroup of the update would reduce the partial sums again) have
- * both launched here; the caller's calls are the same. */
+ * both launched here; the caller's calls are the same.  defer non-zero: the update is
+ * mi_adamw_step_capturable_rows or mi_adamw_step_fused_chain_rows, whose first launch then
+ * finishes the norm for a set of any size (several such calls may follow one norm pass). */
 int mi_adamw_grad_norm_block(const mi_adamw_tensor *d_tensors, const mi_adamw_chunk *d_chunks,
                              int64_t n_chunks, int64_t chunk_elems, float grad_prescale,
-                             float max_norm, mi_adamw_norm_block *d_block, float *d_norm,
-                             void *stream);
+                             float max_norm, int32_t defer, mi_adamw_norm_block *d_block,
+                             float *d_norm, void *stream);
 int mi_adamw_grad_norm_block_flat(const float *d_grad, int64_t n, int64_t chunk_elems,
                                   float grad_prescale, float max_norm,
                                   mi_adamw_norm_block *d_block, float *d_norm, void *stream);

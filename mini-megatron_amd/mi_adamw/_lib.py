@@ -46,6 +46,7 @@ F_BF16_COPY = 1 << 1
 F_WRITE_GRAD = 1 << 2
 F_AMSGRAD = 1 << 3
 F_NORM_BLOCK = 1 << 4
+F_ADVANCE = 1 << 5
 
 T_VEC = 1 << 0
 
@@ -170,7 +171,8 @@ _SIGNATURES = {
     "mi_adamw_build_chunks": ([_vp, _i32, _i64, _vp, _i64], _i64),
     "mi_adamw_grad_norm": ([_vp, _vp, _i64, _i64, _f32, _vp, _vp, _vp, _vp], ctypes.c_int),
     "mi_adamw_grad_norm_flat": ([_vp, _i64, _i64, _f32, _vp, _vp, _vp, _vp], ctypes.c_int),
-    "mi_adamw_grad_norm_block": ([_vp, _vp, _i64, _i64, _f32, _f32, _vp, _vp, _vp], ctypes.c_int),
+    "mi_adamw_grad_norm_block": ([_vp, _vp, _i64, _i64, _f32, _f32, _i32, _vp, _vp, _vp],
+                                 ctypes.c_int),
     "mi_adamw_grad_norm_block_flat": ([_vp, _i64, _i64, _f32, _f32, _vp, _vp, _vp], ctypes.c_int),
     "mi_adamw_grad_norm_flat_noalloc": ([_vp, _i64, _i64, _f32, _vp, _vp, _vp], ctypes.c_int),
     "mi_adamw_grad_sumsq": ([_vp, _vp, _i64, _i64, _f32, _vp, _vp, _vp], ctypes.c_int),

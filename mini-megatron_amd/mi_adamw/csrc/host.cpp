@@ -56,7 +56,7 @@ struct Api {
     int (*set_grads)(mi_adamw_tensor*, int32_t, int32_t, const int32_t*, const uint64_t*,
                      const uint8_t*, void*) = nullptr;
     int (*grad_norm_block)(const mi_adamw_tensor*, const mi_adamw_chunk*, int64_t, int64_t,
-                           float, float, mi_adamw_norm_block*, float*, void*) = nullptr;
+                           float, float, int32_t, mi_adamw_norm_block*, float*, void*) = nullptr;
     int (*grad_norm_block_flat)(const float*, int64_t, int64_t, float, float,
                                 mi_adamw_norm_block*, float*, void*) = nullptr;
     int (*step_prescaled)(const mi_adamw_tensor*, const mi_adamw_chunk*, int64_t, int64_t,
@@ -475,7 +475,7 @@ PyObject* py_norm(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     if (PyErr_Occurred()) return nullptr;
     const int rc =
         pl->tables ? g_api.grad_norm_block(pl->d_rows, pl->d_chunks, pl->n_chunks,
-                                           pl->chunk_elems, pl->prescale, pl->max_norm,
+                                           pl->chunk_elems, pl->prescale, pl->max_norm, 0,
                                            pl->block, norm, s)
                    : g_api.grad_norm_block_flat(pl->flat_row.grad, pl->flat_row.numel,
                                                 pl->chunk_elems, pl->prescale, pl->max_norm,

@@ -379,9 +379,11 @@ struct CaptHyper {
     const float* steps;
     const int32_t* step_index;
     __device__ __forceinline__ ElemScalars get(const mi_adamw_tensor& t, int32_t row) const {
-        const mi_adamw_capt_hyper& c = cp.h[t.hyper];
         const int32_t slot = *((const CONSTANT int32_t*)(step_index) + row);
-        const float step = *((const CONSTANT float*)(steps) + slot);
+        return at(t, *((const CONSTANT float*)(steps) + slot));
+    }
+    __device__ __forceinline__ ElemScalars at(const mi_adamw_tensor& t, float step) const {
+        const mi_adamw_capt_hyper& c = cp.h[t.hyper];
         const float bc1 = 1.0f - powf(c.beta1, step);                 // adam.py:488
         const float bc2 = 1.0f - powf(c.beta2, step);                 // adam.py:497
         float lr = c.lr;
@@ -420,13 +422,7 @@ struct alignas(16) RowScalars {
 };
 static_assert(sizeof(RowScalars) == MI_ADAMW_ROW_SCALAR_BYTES, "one row's values per slot");
 
-__global__ __launch_bounds__(256) void mi_adamw_capt_rows_kernel(
-    const mi_adamw_tensor* __restrict__ rows, int32_t n_rows, CaptHyper hs,
-    RowScalars* __restrict__ out) {
-    const int32_t r = blockIdx.x * 256 + threadIdx.x;
-    if (r >= n_rows) return;
-    out[r].s = hs.get(rows[r], r);
-}
+__device__ __forceinline__ void put_row(RowScalars* out, const ElemScalars& s) { out->s = s; }
 
 struct CaptRowsHyper {
     using Scalars = ElemScalars;
@@ -496,11 +492,15 @@ struct FusedHyper {
     const float* steps;
     const int32_t* step_index;
     __device__ __forceinline__ Scalars get(const mi_adamw_tensor& t, int32_t row) const {
+        if (!kDevSteps) return at(t, 0.0f);
+        const int32_t slot = *((const CONSTANT int32_t*)(step_index) + row);
+        return at(t, *((const CONSTANT float*)(steps) + slot));
+    }
+    __device__ __forceinline__ Scalars at(const mi_adamw_tensor& t, float device_step) const {
         const FusedSet& c = fp.h[t.hyper];
         float bc1 = c.bc1, bc2_sqrt = c.bc2_sqrt;
         if (kDevSteps) {
-            const int32_t slot = *((const CONSTANT int32_t*)(step_index) + row);
-            const double step = *((const CONSTANT float*)(steps) + slot);
+            const double step = device_step;
             bc1 = static_cast<float>(1.0 - pow_f64(c.beta1, step));
             bc2_sqrt = static_cast<float>(sqrt(1.0 - pow_f64(c.beta2, step)));
         }
@@ -543,19 +543,14 @@ struct FusedRow {
 };
 static_assert(sizeof(FusedRow) <= MI_ADAMW_ROW_SCALAR_BYTES, "one row's values per slot");
 
-__global__ __launch_bounds__(256) void mi_adamw_fused_rows_kernel(
-    const mi_adamw_tensor* __restrict__ rows, int32_t n_rows, FusedHyper<true> hs,
-    RowScalars* __restrict__ out) {
-    const int32_t r = blockIdx.x * 256 + threadIdx.x;
-    if (r >= n_rows) return;
-    const FusedScalarsT<false> s = hs.get(rows[r], r);
+__device__ __forceinline__ void put_row(RowScalars* out, const FusedScalarsT<false>& s) {
     FusedRow f;
     f.lr_wd = s.lr_wd;
     f.step_size = s.step_size;
     f.bc2_sqrt = s.bc2_sqrt;
     f.inv_bc2_sqrt = 1.0f / s.bc2_sqrt;
     f.unused = 0.0f;
-    memcpy(&out[r], &f, sizeof(f));
+    memcpy(out, &f, sizeof(f));
 }
 
 struct FusedRowsHyper {
@@ -803,6 +798,40 @@ __global__ __launch_bounds__(kNormThreads) void mi_adamw_norm_finalize_kernel(
         const float norm = static_cast<float>(__builtin_sqrt(s));
         *norm_out = norm;
         *coef_out = clip_coef(norm, max_norm);
+    }
+}
+
+// The launch before an update with device step counts: one thread per table row forms the
+// row's per-step values (HS::at, the code an update forming them itself runs), after adding
+// 1 to the row's step count if `advance`.  With a norm block whose partial sums still wait,
+// one workgroup more reduces them.  One launch of a few microseconds does what would
+// otherwise be three (increment, finalize, rows): 5.4M parameters, clip, as a replayed graph
+// 48.2 -> 40.5 us.
+template <class HS>
+__global__ __launch_bounds__(kNormThreads) void mi_adamw_rows_kernel(
+    const mi_adamw_tensor* __restrict__ rows, int32_t n_rows, HS hs,
+    RowScalars* __restrict__ out, float* __restrict__ advance, mi_adamw_norm_block* block) {
+    if (block && blockIdx.x == gridDim.x - 1) {
+        const int32_t n = block->n_partials;
+        if (n == 0) return;
+        const double s = sum_partials<kNormThreads>(block->partials, n);
+        if (threadIdx.x == 0) {
+            const float norm = static_cast<float>(__builtin_sqrt(s));
+            *block->norm = norm;
+            block->coef = clip_coef(norm, block->max_norm);
+            block->n_partials = 0;
+        }
+        return;
+    }
+    const int32_t r = blockIdx.x * kNormThreads + threadIdx.x;
+    if (r >= n_rows) return;
+    if (advance) {
+        float* step = advance + hs.step_index[r];
+        const float next = *step + 1.0f;
+        *step = next;
+        put_row(out + r, hs.at(rows[r], next));
+    } else {
+        put_row(out + r, hs.get(rows[r], r));
     }
 }
 
@@ -1214,10 +1243,11 @@ int launch_norm(const Src& src, int64_t n_chunks, int64_t chunk_elems, float max
 // Pass 1 into a norm block, the rest left to the update or, for a large set, finalized here.
 template <class Src>
 int launch_norm_block(const Src& src, int64_t n_chunks, int64_t chunk_elems, float pre,
-                      float max_norm, mi_adamw_norm_block* block, float* norm, hipStream_t s) {
+                      float max_norm, bool defer, mi_adamw_norm_block* block, float* norm,
+                      hipStream_t s) {
     if (!block || !norm || !aligned(block, 8) || !finite(pre)) return MI_ADAMW_E_INVALID;
     if (n_chunks <= 0 || !chunk_elems_ok(chunk_elems)) return MI_ADAMW_E_INVALID;
-    const bool fold = n_chunks <= kFoldElems / chunk_elems;
+    const bool fold = defer || n_chunks <= kFoldElems / chunk_elems;
     const unsigned n = grid_for(n_chunks, kNormBlocks, kNormThreads);
     const BlockArgs ba{block, norm, max_norm, fold ? static_cast<int32_t>(n) : 0};
     unsigned grid = 0;
@@ -1281,19 +1311,26 @@ int launch_update_cw(const Src& src, int64_t n_chunks, int64_t chunk_elems, cons
     return MI_ADAMW_E_INVALID;
 }
 
+// Whether launch_update takes these arguments.
+bool update_args_ok(int64_t n_chunks, int64_t chunk_elems, const float* scale,
+                    int32_t state_dtype, int32_t flags) {
+    if (n_chunks <= 0 || !chunk_elems_ok(chunk_elems)) return false;
+    if (state_dtype != MI_ADAMW_STATE_F32 && state_dtype != MI_ADAMW_STATE_BF16) return false;
+    if (flags & ~(MI_ADAMW_F_CLIP | MI_ADAMW_F_BF16_COPY | MI_ADAMW_F_WRITE_GRAD |
+                  MI_ADAMW_F_AMSGRAD | MI_ADAMW_F_NORM_BLOCK))
+        return false;
+    const bool block = flags & MI_ADAMW_F_NORM_BLOCK;
+    if ((flags & MI_ADAMW_F_CLIP) ? !scale : block) return false;
+    return !block || aligned(scale, 8);
+}
+
 template <class Src, class HS>
 int launch_update(const Src& src, int64_t n_chunks, int64_t chunk_elems, const HS& hs,
                   const float* scale, int32_t state_dtype, int32_t flags, int32_t max_blocks,
                   hipStream_t s, float pre = 1.0f) {
-    if (n_chunks <= 0 || !chunk_elems_ok(chunk_elems)) return MI_ADAMW_E_INVALID;
-    if (state_dtype != MI_ADAMW_STATE_F32 && state_dtype != MI_ADAMW_STATE_BF16)
-        return MI_ADAMW_E_INVALID;
-    if (flags & ~(MI_ADAMW_F_CLIP | MI_ADAMW_F_BF16_COPY | MI_ADAMW_F_WRITE_GRAD |
-                  MI_ADAMW_F_AMSGRAD | MI_ADAMW_F_NORM_BLOCK))
+    if (!update_args_ok(n_chunks, chunk_elems, scale, state_dtype, flags))
         return MI_ADAMW_E_INVALID;
     const bool clip = flags & MI_ADAMW_F_CLIP, block = flags & MI_ADAMW_F_NORM_BLOCK;
-    if (clip ? !scale : block) return MI_ADAMW_E_INVALID;
-    if (block && !aligned(scale, 8)) return MI_ADAMW_E_INVALID;
 #define MI_ADAMW_CLIP(S)                                                                       \
     (block  ? launch_update_cw<Src, HS, S, kBlock>(src, n_chunks, chunk_elems, hs, scale, pre, \
                                                    flags, max_blocks, s)                       \
@@ -1303,6 +1340,20 @@ int launch_update(const Src& src, int64_t n_chunks, int64_t chunk_elems, const H
                                                     pre, flags, max_blocks, s))
     return state_dtype == MI_ADAMW_STATE_F32 ? MI_ADAMW_CLIP(float) : MI_ADAMW_CLIP(uint16_t);
 #undef MI_ADAMW_CLIP
+}
+
+// The launch before an update with device step counts.
+template <class HS>
+int launch_rows(const mi_adamw_tensor* d_tensors, int32_t n_rows, const HS& hs, RowScalars* rows,
+                const float* scale, int32_t flags, hipStream_t s) {
+    mi_adamw_norm_block* block = nullptr;
+    if (flags & MI_ADAMW_F_NORM_BLOCK)
+        block = reinterpret_cast<mi_adamw_norm_block*>(const_cast<float*>(scale));
+    float* advance = (flags & MI_ADAMW_F_ADVANCE) ? const_cast<float*>(hs.steps) : nullptr;
+    hipLaunchKernelGGL(mi_adamw_rows_kernel<HS>,
+                       dim3((n_rows + kNormThreads - 1) / kNormThreads + (block ? 1 : 0)),
+                       dim3(kNormThreads), 0, s, d_tensors, n_rows, hs, rows, advance, block);
+    return launch_status();
 }
 
 // The memory-only twin of launch_update (no clip: the gradient is read either way).
@@ -1504,12 +1555,12 @@ int mi_adamw_grad_norm_flat(const float* d_grad, int64_t n, int64_t chunk_elems,
 
 int mi_adamw_grad_norm_block(const mi_adamw_tensor* d_tensors, const mi_adamw_chunk* d_chunks,
                              int64_t n_chunks, int64_t chunk_elems, float grad_prescale,
-                             float max_norm, mi_adamw_norm_block* d_block, float* d_norm,
-                             void* stream) {
+                             float max_norm, int32_t defer, mi_adamw_norm_block* d_block,
+                             float* d_norm, void* stream) {
     if (!d_tensors || !d_chunks) return MI_ADAMW_E_INVALID;
     TableSource src{d_tensors, d_chunks};
-    return launch_norm_block(src, n_chunks, chunk_elems, grad_prescale, max_norm, d_block, d_norm,
-                             static_cast<hipStream_t>(stream));
+    return launch_norm_block(src, n_chunks, chunk_elems, grad_prescale, max_norm, defer != 0,
+                             d_block, d_norm, static_cast<hipStream_t>(stream));
 }
 
 int mi_adamw_grad_norm_block_flat(const float* d_grad, int64_t n, int64_t chunk_elems,
@@ -1521,8 +1572,8 @@ int mi_adamw_grad_norm_block_flat(const float* d_grad, int64_t n, int64_t chunk_
     src.t.grad = const_cast<float*>(d_grad);
     src.t.numel = n;
     const int64_t n_chunks = (n + chunk_elems - 1) / chunk_elems;
-    return launch_norm_block(src, n_chunks, chunk_elems, grad_prescale, max_norm, d_block, d_norm,
-                             static_cast<hipStream_t>(stream));
+    return launch_norm_block(src, n_chunks, chunk_elems, grad_prescale, max_norm, false, d_block,
+                             d_norm, static_cast<hipStream_t>(stream));
 }
 
 int mi_adamw_grad_norm_flat_noalloc(const float* d_grad, int64_t n, int64_t chunk_elems,
@@ -1703,17 +1754,17 @@ int mi_adamw_step_capturable_rows(const mi_adamw_tensor* d_tensors, int32_t n_ro
                                   int32_t max_blocks, void* stream) {
     CaptHyper hs;
     if (!d_tensors || n_rows <= 0 || !d_chunks || !d_row_scalars || !aligned(d_row_scalars, 16) ||
-        capt_hyper_from(hypers, n_hyper, d_steps, d_step_index, hs))
+        capt_hyper_from(hypers, n_hyper, d_steps, d_step_index, hs) ||
+        !update_args_ok(n_chunks, chunk_elems, d_grad_scale, state_dtype,
+                        flags & ~MI_ADAMW_F_ADVANCE))
         return MI_ADAMW_E_INVALID;
     const hipStream_t s = static_cast<hipStream_t>(stream);
     RowScalars* rows = static_cast<RowScalars*>(d_row_scalars);
-    hipLaunchKernelGGL(mi_adamw_capt_rows_kernel, dim3((n_rows + 255) / 256), dim3(256), 0, s,
-                       d_tensors, n_rows, hs, rows);
-    const int rc = launch_status();
+    const int rc = launch_rows(d_tensors, n_rows, hs, rows, d_grad_scale, flags, s);
     if (rc) return rc;
     TableSource src{d_tensors, d_chunks};
     return launch_update(src, n_chunks, chunk_elems, CaptRowsHyper{rows}, d_grad_scale,
-                         state_dtype, flags, max_blocks, s);
+                         state_dtype, flags & ~MI_ADAMW_F_ADVANCE, max_blocks, s);
 }
 
 int mi_adamw_step_fused_chain(const mi_adamw_tensor* d_tensors, const mi_adamw_chunk* d_chunks,
@@ -1754,7 +1805,9 @@ int mi_adamw_step_fused_chain_rows(const mi_adamw_tensor* d_tensors, int32_t n_r
                                    void* stream) {
     if (!d_tensors || n_rows <= 0 || !d_chunks || !hypers || n_hyper <= 0 ||
         n_hyper > MI_ADAMW_MAX_HYPER || !finite(grad_prescale) || !d_steps || !d_step_index ||
-        !d_row_scalars || !aligned(d_row_scalars, 16))
+        !d_row_scalars || !aligned(d_row_scalars, 16) ||
+        !update_args_ok(n_chunks, chunk_elems, d_grad_scale, state_dtype,
+                        flags & ~MI_ADAMW_F_ADVANCE))
         return MI_ADAMW_E_INVALID;
     FusedHyper<true> hs;
     memset(&hs, 0, sizeof(hs));
@@ -1763,17 +1816,15 @@ int mi_adamw_step_fused_chain_rows(const mi_adamw_tensor* d_tensors, int32_t n_r
     hs.step_index = d_step_index;
     const hipStream_t s = static_cast<hipStream_t>(stream);
     RowScalars* rows = static_cast<RowScalars*>(d_row_scalars);
-    hipLaunchKernelGGL(mi_adamw_fused_rows_kernel, dim3((n_rows + 255) / 256), dim3(256), 0, s,
-                       d_tensors, n_rows, hs, rows);
-    const int rc = launch_status();
+    const int rc = launch_rows(d_tensors, n_rows, hs, rows, d_grad_scale, flags, s);
     if (rc) return rc;
     FusedRowsHyper rh;
     memset(&rh, 0, sizeof(rh));
     rh.fp = hs.fp;
     rh.rows = rows;
     TableSource src{d_tensors, d_chunks};
-    return launch_update(src, n_chunks, chunk_elems, rh, d_grad_scale, state_dtype, flags,
-                         max_blocks, s, grad_prescale);
+    return launch_update(src, n_chunks, chunk_elems, rh, d_grad_scale, state_dtype,
+                         flags & ~MI_ADAMW_F_ADVANCE, max_blocks, s, grad_prescale);
 }
 
 int mi_adamw_step_flat_fused_chain(const mi_adamw_tensor* t, const mi_adamw_fused_hyper* hyper,

@@ -877,12 +877,15 @@ class FusedAdamW(Optimizer):
                 self._init_vmax(rec.p, st)
 
         if self.capturable:
-            # step_t += 1 on the device (adam.py:414), one op for every param with a
-            # grad; one constant set per group, the kernel forms the per-step values
-            if len(entries) == len(self._step_views):
-                self._steps.add_(1)
-            else:
-                self._steps.index_add_(0, *self._step_increment(entries, device))
+            # step_t += 1 on the device (adam.py:414) for every param with a grad, by the
+            # launch that forms the rows' per-step values; an empty param has no row, so
+            # with one of those it is an op of its own.  One constant set per group.
+            advance = all(rec.p.numel() for rec, _ in entries)
+            if not advance:
+                if len(entries) == len(self._step_views):
+                    self._steps.add_(1)
+                else:
+                    self._steps.index_add_(0, *self._step_increment(entries, device))
             gis = sorted({rec.gi for rec, _ in entries})
             remap = {gi: i for i, gi in enumerate(gis)}
             hyper_idx = [remap[rec.gi] for rec, _ in entries]
@@ -923,7 +926,8 @@ class FusedAdamW(Optimizer):
 
         with torch.cuda.device(device):
             self._launch(entries, hyper_idx, hypers, hyper_ams, hyper_fused, device,
-                         None if self.capturable else hyper_group)
+                         None if self.capturable else hyper_group,
+                         _lib.F_ADVANCE if self.capturable and advance else 0)
         if self._copy_sync is not None:
             # the launch wrote these masters' copies
             for rec, _ in entries:
@@ -1224,7 +1228,7 @@ class FusedAdamW(Optimizer):
                               hyper=0, flags=int(r["flags"]))
 
     def _launch(self, entries, hyper_idx, hypers, hyper_ams, hyper_fused, device,
-                hyper_group: list | None = None) -> None:
+                hyper_group: list | None = None, advance: int = 0) -> None:
         lib = _lib.load()
         self._fast = None
         stream = torch.cuda.current_stream(device).cuda_stream
@@ -1294,7 +1298,7 @@ class FusedAdamW(Optimizer):
             if norm_launch.n_chunks == 0:
                 # nothing but empty tensors: torch's norm of no elements is 0
                 norm.zero_()
-            elif norm_launch.n_rows == 1:
+            elif norm_launch.n_rows == 1 and not self.capturable:
                 row = self._row_struct(norm_launch)
                 _lib.check(lib.mi_adamw_grad_norm_block_flat(
                     row.grad, row.numel, self.chunk_elems, self.grad_prescale,
@@ -1304,8 +1308,8 @@ class FusedAdamW(Optimizer):
                 _lib.check(lib.mi_adamw_grad_norm_block(
                     norm_launch.rows.data_ptr(), norm_launch.chunks.data_ptr(),
                     norm_launch.n_chunks, self.chunk_elems, self.grad_prescale,
-                    float(self.max_grad_norm), norm_block.data_ptr(), norm.data_ptr(), stream),
-                    "mi_adamw_grad_norm_block")
+                    float(self.max_grad_norm), self.capturable, norm_block.data_ptr(),
+                    norm.data_ptr(), stream), "mi_adamw_grad_norm_block")
             self.last_grad_norm = norm
             flags |= _lib.F_CLIP | _lib.F_NORM_BLOCK
             if self.clip_write_grads:
@@ -1314,7 +1318,7 @@ class FusedAdamW(Optimizer):
         for launch, (_, _, hs, (ams, fused), _) in zip(launches, parts):
             if launch.n_chunks == 0:
                 continue
-            lflags = flags | (_lib.F_AMSGRAD if ams else 0)
+            lflags = flags | advance | (_lib.F_AMSGRAD if ams else 0)
             if fused:
                 self._launch_fused_chain(launch, hs, norm_block, state_code, lflags, stream)
                 continue

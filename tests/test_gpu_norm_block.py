@@ -71,3 +71,29 @@ def test_norm_of_a_recorded_step(dev, n):
         norm = np.float32(opt.last_grad_norm.item())
         assert norm == O.total_norm([p.grad.cpu().numpy()])
         (torch.ones(4096, device=dev) * 3).sum().item()     # other work between the replays
+
+
+@pytest.mark.parametrize("fused", [False, True])
+@pytest.mark.parametrize("sizes", [(3, 70), (5, 0, 4099), (300, 1) * 150, (FOLD, 4097)])
+def test_device_step_counts_and_norm(dev, sizes, fused):
+    """capturable=True: the launch before the update advances the counts (an empty tensor's,
+    which has no row, apart), forms the rows and finishes the norm; more than 256 rows take
+    several of its workgroups."""
+    import mi_adamw
+    gen = torch.Generator(device=dev).manual_seed(len(sizes))
+    values = [torch.randn(n, device=dev, generator=gen) for n in sizes]
+    ours = [torch.nn.Parameter(v.clone()) for v in values]
+    ref = [torch.nn.Parameter(v.clone()) for v in values]
+    hp = dict(lr=1e-2, capturable=True, fused=fused or None)
+    opt = mi_adamw.FusedAdamW(ours, max_grad_norm=0.5, **hp)
+    topt = torch.optim.AdamW(ref, foreach=None if fused else False, **hp)
+    for k in range(4):
+        for i, (q, r) in enumerate(zip(ours, ref)):
+            g = torch.randn(q.numel(), device=dev, generator=gen)
+            q.grad, r.grad = (g, g.clone()) if i or k != 2 else (None, None)
+        opt.step()
+        torch.nn.utils.clip_grads_with_norm_(ref, 0.5, opt.last_grad_norm.clone())
+        topt.step()
+        for q, r in zip(ours, ref):
+            assert max_ulp(q, r) == 0
+            assert float(opt.state[q]["step"]) == float(topt.state[r]["step"])
