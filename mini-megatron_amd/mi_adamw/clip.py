@@ -12,6 +12,8 @@ coefficient on the device) and an in-place scale pass.  Use
 """
 from __future__ import annotations
 
+import threading
+
 import numpy as np
 import torch
 
@@ -20,6 +22,8 @@ from . import _lib
 _CHUNK = 4096
 _workspace: dict[tuple, tuple] = {}
 _cache: dict[tuple, tuple] = {}
+# threads that share a stream share its tables: one call's patch and passes at a time
+_lock = threading.Lock()
 
 
 def _ws(device, stream: int):
@@ -54,7 +58,7 @@ def _tables(grads, device, stream: int):
     rows["numel"] = [g.numel() * (2 if torch.is_complex(g) else 1) for g in grads]
     rows["flags"] = np.where(ptrs % 16 == 0, _lib.T_VEC, 0)
     rows = rows[rows["numel"] > 0]
-    key = (device, stream, tuple(int(n) for n in rows["numel"]))
+    key = (device, stream, rows["numel"].tobytes())
     launch = _cache.get(key)
     if launch is not None:
         if not np.array_equal(launch.host_rows["grad"], rows["grad"]):
@@ -67,33 +71,43 @@ def _tables(grads, device, stream: int):
     return launch
 
 
-@torch.no_grad()
-def clip_grad_norm_(parameters, max_norm: float, norm_type: float = 2.0,
-                    error_if_nonfinite: bool = False, foreach: bool | None = None) -> torch.Tensor:
-    """Clip the global gradient norm in place; returns the total norm (0-d tensor)."""
-    if isinstance(parameters, torch.Tensor):
-        parameters = [parameters]
-    grads = [p.grad for p in parameters if p.grad is not None]
-    if float(norm_type) != 2.0:
-        raise NotImplementedError("mi_adamw.clip_grad_norm_ supports norm_type=2 only")
-    if len(grads) == 0:
-        return torch.tensor(0.0)
-    device = grads[0].device
-    for g in grads:
-        if g.device != device or g.device.type != "cuda":
-            raise RuntimeError("mi_adamw.clip_grad_norm_ needs every gradient on one ROCm GPU")
-        if g.dtype not in (torch.float32, torch.complex64) or not g.is_contiguous() or g.is_sparse:
-            raise NotImplementedError("mi_adamw.clip_grad_norm_ supports dense contiguous fp32 "
-                                      "gradients only")
-    lib = _lib.load()
-    norm = torch.empty((), dtype=torch.float32, device=device)
-    with torch.cuda.device(device):
-        stream = torch.cuda.current_stream(device).cuda_stream
-        launch = _tables(grads, device, stream)
+def _move(launch, ptrs: bytes, device) -> None:
+    """The gradients lie elsewhere than the launch's table says: the table is patched in
+    place (it belongs to one stream), or replaced if a graph has recorded its address."""
+    grads = np.frombuffer(ptrs, dtype=np.uint64)
+    rows = launch.host_rows.copy()
+    idx = np.flatnonzero(grads != rows["grad"]).astype(np.int32)
+    rows["param"] = rows["grad"] = grads
+    rows["flags"] = np.where(grads % 16 == 0, _lib.T_VEC, 0)
+    if launch.recorded:
+        launch.set_rows(rows, device)
+        return
+    new = np.ascontiguousarray(grads[idx])
+    vec = (new % 16 == 0).astype(np.uint8)
+    code = _lib.load().mi_adamw_set_grads(
+        launch.rows.data_ptr(), launch.n_rows, len(idx), idx.ctypes.data, new.ctypes.data,
+        vec.ctypes.data, torch._C._cuda_getCurrentRawStream(device.index))
+    if code != _lib.OK:
+        _cache.clear()      # the device table may hold part of the patch
+    _lib.check(code, "mi_adamw_set_grads")
+    launch.host_rows = rows
+
+
+def _run(launch, ptrs: bytes | None, device, stream: int, max_norm: float, norm_type: float,
+         error_if_nonfinite: bool) -> torch.Tensor:
+    """The norm and scale passes over a launch's tables; `ptrs`: where the gradients are
+    (None: where the tables say)."""
+    if torch._C._cuda_getDevice() != device.index:
+        with torch.cuda.device(device):
+            return _run(launch, ptrs, device, stream, max_norm, norm_type, error_if_nonfinite)
+    with _lock:
+        if torch._C._cuda_isCurrentStreamCapturing():
+            launch.recorded = True
+        if ptrs is not None and ptrs != launch.host_rows["grad"].tobytes():
+            _move(launch, ptrs, device)
+        lib = _lib.load()
+        norm = torch.empty((), dtype=torch.float32, device=device)
         partials, coef = _ws(device, stream)
-        if launch.n_chunks == 0:
-            norm.zero_()
-            return norm
         _lib.check(lib.mi_adamw_grad_norm(
             launch.rows.data_ptr(), launch.chunks.data_ptr(), launch.n_chunks, _CHUNK,
             float(max_norm), partials.data_ptr(), norm.data_ptr(),
@@ -107,4 +121,40 @@ def clip_grad_norm_(parameters, max_norm: float, norm_type: float = 2.0,
         _lib.check(lib.mi_adamw_scale_grads(
             launch.rows.data_ptr(), launch.chunks.data_ptr(), launch.n_chunks, _CHUNK,
             coef.data_ptr(), stream), "mi_adamw_scale_grads")
-    return norm
+        return norm
+
+
+@torch.no_grad()
+def clip_grad_norm_(parameters, max_norm: float, norm_type: float = 2.0,
+                    error_if_nonfinite: bool = False, foreach: bool | None = None) -> torch.Tensor:
+    """Clip the global gradient norm in place; returns the total norm (0-d tensor)."""
+    parameters = [parameters] if isinstance(parameters, torch.Tensor) else list(parameters)
+    if _lib._host is not None and float(norm_type) == 2.0:
+        found = _lib._host.grads(parameters, torch.Tensor, torch.nn.Parameter)
+        if found is not None:
+            index, numels, ptrs = found
+            stream = torch._C._cuda_getCurrentRawStream(index)
+            device = torch.device("cuda", index)
+            launch = _cache.get((device, stream, numels))
+            if launch is not None:
+                return _run(launch, ptrs, device, stream, max_norm, norm_type,
+                            error_if_nonfinite)
+    grads = [p.grad for p in parameters if p.grad is not None]
+    if float(norm_type) != 2.0:
+        raise NotImplementedError("mi_adamw.clip_grad_norm_ supports norm_type=2 only")
+    if len(grads) == 0:
+        return torch.tensor(0.0)
+    device = grads[0].device
+    for g in grads:
+        if g.device != device or g.device.type != "cuda":
+            raise RuntimeError("mi_adamw.clip_grad_norm_ needs every gradient on one ROCm GPU")
+        if g.dtype not in (torch.float32, torch.complex64) or not g.is_contiguous() or g.is_sparse:
+            raise NotImplementedError("mi_adamw.clip_grad_norm_ supports dense contiguous fp32 "
+                                      "gradients only")
+    _lib.load()
+    with torch.cuda.device(device):
+        stream = torch.cuda.current_stream(device).cuda_stream
+        launch = _tables(grads, device, stream)
+        if launch.n_chunks == 0:
+            return torch.zeros((), dtype=torch.float32, device=device)
+    return _run(launch, None, device, stream, max_norm, norm_type, error_if_nonfinite)

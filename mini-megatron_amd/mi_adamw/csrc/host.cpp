@@ -27,7 +27,9 @@
 //   update(plan, stream, hypers, n) -> int   mi_adamw_step*_prescaled, or with the
 //                                       fused=True chain mi_adamw_step*_fused_chain
 //   sync_versions(plan, dict)           dict[id(p)] = (p._version, p.data_ptr())
+//   grads(params, ...)                  what clip_grad_norm_ needs of its gradients
 
+#define PY_SSIZE_T_CLEAN
 #include <Python.h>
 
 #include <ATen/core/Tensor.h>
@@ -556,6 +558,56 @@ PyObject* sync_versions(Plan* pl, PyObject* dict) {
     Py_RETURN_NONE;
 }
 
+// grads(params, tensor_type, parameter_type) -> (device index, numels, pointers) or None
+// The gradients of a list of parameters as clip_grad_norm_'s tables take them: the element
+// counts (complex ones twice) and addresses, int64 and uint64 in two bytes objects, empty
+// gradients left out.  None for whatever its Python path has to look at: no gradient with
+// elements, another device than the first one's or no GPU, another dtype, a strided or sparse
+// one, no storage, an object that is no plain tensor or parameter, or a tensor whose .grad
+// autograd does not keep.
+PyObject* grads(PyObject* params, PyObject* tensor_type, PyObject* parameter_type) {
+    const Py_ssize_t n = PyList_GET_SIZE(params);
+    std::vector<int64_t> numel;
+    std::vector<uint64_t> ptr;
+    numel.reserve(n);
+    ptr.reserve(n);
+    c10::Device device(c10::DeviceType::CPU);
+    for (Py_ssize_t i = 0; i < n; ++i) {
+        PyObject* o = PyList_GET_ITEM(params, i);
+        PyObject* type = reinterpret_cast<PyObject*>(Py_TYPE(o));
+        if ((type != tensor_type && type != parameter_type) || !is_tensor(o)) Py_RETURN_NONE;
+        const at::Tensor& p = THPVariable_Unpack(o);
+        if (!p.is_leaf()) Py_RETURN_NONE;
+        const at::Tensor& g = p.grad();
+        if (!g.defined()) continue;
+        if (device.is_cpu()) device = g.device();
+        if (!device.is_cuda() || g.device() != device || g.layout() != c10::kStrided ||
+            (g.scalar_type() != at::kFloat && g.scalar_type() != at::kComplexFloat) ||
+            !g.is_contiguous())
+            Py_RETURN_NONE;
+        if (g.numel() == 0) continue;
+        numel.push_back(g.numel() * (g.scalar_type() == at::kComplexFloat ? 2 : 1));
+        ptr.push_back(reinterpret_cast<uint64_t>(g.data_ptr()));
+    }
+    if (numel.empty()) Py_RETURN_NONE;
+    const Py_ssize_t bytes = static_cast<Py_ssize_t>(numel.size() * 8);
+    return Py_BuildValue("(iy#y#)", static_cast<int>(device.index()),
+                         reinterpret_cast<const char*>(numel.data()), bytes,
+                         reinterpret_cast<const char*>(ptr.data()), bytes);
+}
+
+PyObject* py_grads(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+    if (nargs != 3 || !PyList_CheckExact(args[0])) {
+        PyErr_SetString(PyExc_TypeError, "grads(list, tensor type, parameter type)");
+        return nullptr;
+    }
+    try {
+        return grads(args[0], args[1], args[2]);
+    } catch (const std::exception&) {
+        Py_RETURN_NONE;     // an accessor refused a tensor: the Python path reports it
+    }
+}
+
 PyMethodDef kMethods[] = {
     {"bind", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(py_bind)), METH_FASTCALL,
      "bind the library's entry points"},
@@ -571,6 +623,8 @@ PyMethodDef kMethods[] = {
     {"sync_versions",
      reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(py_sync_versions)), METH_FASTCALL,
      "record every parameter's version and address"},
+    {"grads", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(py_grads)),
+     METH_FASTCALL, "element counts and addresses of a parameter list's gradients"},
     {nullptr, nullptr, 0, nullptr}};
 
 PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_host",

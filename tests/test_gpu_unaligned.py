@@ -24,7 +24,9 @@ MARK = -7.0     # exact in bf16
 def dev():
     if not torch.cuda.is_available():
         pytest.fail("GPU test run without a ROCm GPU")
-    return torch.device("cuda", 0)
+    yield torch.device("cuda", 0)
+    from mi_adamw import clip
+    clip._cache.clear()      # other tests count the tables of their own sizes
 
 
 def _guarded(values: torch.Tensor, offset: int):
