@@ -1082,7 +1082,7 @@ void mi_adamw_update_kernel(
 // ---------------------------------------------------------------------------
 // g *= coef (clip write-back on its own).
 //
-// One stream read and written: one dwordx4 group per lane, 512-thread workgroups, as many
+// One stream read and written: dwordx4 groups, 512-thread workgroups, as many
 // as fit (the table lookup's latency needs them: with six waves per SIMD it is 5% slower),
 // runs of 32 tiles per XCD.  clip_grad_norm_ of 163M gradients, 1024-thread workgroups over
 // 4096 elements in plain order 309 us, in runs of 16 301, this 300; four groups per lane
@@ -1090,13 +1090,25 @@ void mi_adamw_update_kernel(
 // for them (330 us a call).
 // A coefficient of 1 (the norm under its threshold): g * 1 is g, bit for bit (a gradient
 // with a NaN or an infinity gives another coefficient), so the gradients stay unread.
-// 163M gradients under the threshold: clip_grad_norm_ 315 -> 144 us, and a clipped step that
+// 163M gradients under the threshold: clip_grad_norm_ 315 -> 120 us, and a clipped step that
 // stores its gradients, where the update leaves its store out likewise, 996 -> 809.
+//
+// kGroups: dwordx4 groups per lane, both loaded before the first is stored.  What a pass
+// under the threshold costs is starting its waves and ending them, 19 of them per ns, so
+// two groups halve it; over it they cost a set whose last round of workgroups weighs.
+// clip_grad_norm_'s two passes in us, one group and two, under | over the threshold:
+//    17M  20.0  18.3 |  40.0  41.3        90M          | 166.8 167.1
+//    60M             | 112.8 114.3       163M 128.4 112.0 | 294.7 295.2
+//   604M 455.6 394.1 | 1069  1060
+// so two from kScaleTwoElems on (two groups in runs of 8 or 32 tiles instead of 16, in
+// 256-thread workgroups or with half the waves are 0.7-8% slower over it).
 
 constexpr int kScaleThreads = 512;
 constexpr int kScaleTile = kScaleThreads * kVec;
-constexpr int kScaleRun = 32;
+constexpr int kScaleRun = 32;                        // in tiles of one group
+constexpr int64_t kScaleTwoElems = int64_t(80) << 20;
 
+template <int kGroups>
 __global__ __launch_bounds__(kScaleThreads) void mi_adamw_scale_kernel(
     TableSource src, Items items, const float* __restrict__ coef) {
     const float s = *coef;
@@ -1105,15 +1117,21 @@ __global__ __launch_bounds__(kScaleThreads) void mi_adamw_scale_kernel(
         mi_adamw_tensor t;
         int64_t begin, end;
         int32_t row;
-        if (!items.get<kScaleTile>(src, item_order<kScaleRun>(w, items.n), t, begin, end, row))
+        if (!items.get<kScaleTile * kGroups>(src, item_order<kScaleRun / kGroups>(w, items.n), t,
+                                             begin, end, row))
             continue;
         float* __restrict__ G = t.grad;
         const int64_t vend = begin + ((end - begin) & ~static_cast<int64_t>(kVec - 1));
         const int64_t i = begin + threadIdx.x * kVec;
-        if (i < vend) {
-            const f32x4 g = ld4(G + i);
-            st4(G + i, f32x4{g.x * s, g.y * s, g.z * s, g.w * s});
-        }
+        f32x4 g[kGroups];
+#pragma unroll
+        for (int k = 0; k < kGroups; ++k)
+            if (i + k * kScaleTile < vend) g[k] = ld4(G + i + k * kScaleTile);
+#pragma unroll
+        for (int k = 0; k < kGroups; ++k)
+            if (i + k * kScaleTile < vend)
+                st4(G + i + k * kScaleTile,
+                    f32x4{g[k].x * s, g[k].y * s, g[k].z * s, g[k].w * s});
         const int64_t j = vend + threadIdx.x;      // the tensor's last elements, up to three
         if (j < end) st1(G + j, ld1(G + j) * s);
     }
@@ -1671,8 +1689,10 @@ int mi_adamw_scale_grads(const mi_adamw_tensor* d_tensors, const mi_adamw_chunk*
     if (!d_tensors || !d_chunks || !d_coef || n_chunks <= 0 || !chunk_elems_ok(chunk_elems))
         return MI_ADAMW_E_INVALID;
     TableSource src{d_tensors, d_chunks};
-    const Items items = items_of(n_chunks, chunk_elems, kScaleTile);
-    hipLaunchKernelGGL(mi_adamw_scale_kernel, dim3(grid_for(items.n, 0, kScaleThreads)), dim3(kScaleThreads), 0,
+    const bool two = n_chunks >= kScaleTwoElems / chunk_elems;
+    const Items items = items_of(n_chunks, chunk_elems, two ? 2 * kScaleTile : kScaleTile);
+    hipLaunchKernelGGL(two ? mi_adamw_scale_kernel<2> : mi_adamw_scale_kernel<1>,
+                       dim3(grid_for(items.n, 0, kScaleThreads)), dim3(kScaleThreads), 0,
                        static_cast<hipStream_t>(stream), src, items, d_coef);
     return launch_status();
 }

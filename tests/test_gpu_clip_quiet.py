@@ -44,3 +44,27 @@ def test_coefficient_of_one(dev, special, max_norm, step):
         both = torch.isnan(q.grad) & torch.isnan(r.grad)
         assert torch.equal(torch.isnan(q.grad), torch.isnan(r.grad))
         assert torch.equal(_bits(q.grad.masked_fill(both, 0)), _bits(r.grad.masked_fill(both, 0)))
+
+
+@pytest.mark.parametrize("below", [True, False])
+def test_scale_at_the_two_group_rule(dev, below):
+    """Sets on both sides of the size from which a lane of the scale pass takes two groups
+    (80 Mi elements, counted in 4096-element chunks), with tensors that end around its tiles
+    (2048 and 4096 elements) and begin off a 16-byte boundary: g * coef, one fp32 rounding."""
+    import mi_adamw
+    sizes = [1, 3, 2047, 2048, 2049, 2051, 4095, 4096, 4097, 6145, 8191]
+    chunks = (80 << 20) // 4096 - sum(-(-n // 4096) for n in sizes) - (1 if below else 0)
+    sizes.insert(5, chunks * 4096 - 1)
+    block = torch.empty(sum(sizes), device=dev)
+    block.normal_(0.0, 1e-2, generator=torch.Generator(device=dev).manual_seed(9))
+    was = block.clone()
+    params = []
+    for g in block.split(sizes):
+        params.append(torch.nn.Parameter(torch.empty_like(g)))
+        params[-1].grad = g
+    norm = mi_adamw.clip_grad_norm_(params, 1.0)
+    exact = was.double().square().sum().sqrt().item()
+    assert abs(norm.item() - exact) <= 2e-7 * exact      # one fp32 rounding of a float64 sum
+    coef = (1.0 / (norm + 1e-6)).clamp(max=1.0)
+    assert coef.item() < 1.0
+    assert torch.equal(block, was * coef)
