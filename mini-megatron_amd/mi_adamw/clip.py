@@ -6,8 +6,9 @@ between ``loss.backward()`` and ``optimizer.step()`` (main.py:207-209).  This
 function keeps that signature and result: the global L2 norm of every gradient
 as one vector (torch/nn/utils/clip_grad.py:50-117), then
 ``g *= min(max_norm / (norm + 1e-6), 1)`` in place (clip_grad.py:121-183).
-Two launches: the float64 sum-of-squares pass (which also computes the
-coefficient on the device) and an in-place scale pass.  Use
+Three launches: the float64 sum-of-squares pass, a one-workgroup finalize (norm
+and coefficient, on the device) and an in-place scale pass, which leaves the
+gradients alone where the coefficient is 1.  Use
 ``FusedAdamW(max_grad_norm=...)`` instead to fold the scale into the step.
 """
 from __future__ import annotations
