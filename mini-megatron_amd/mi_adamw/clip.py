@@ -19,38 +19,32 @@ import numpy as np
 import torch
 
 from . import _lib
+from .optimizer import _ROW_DTYPE, _Launch
 
 _CHUNK = 4096
-_workspace: dict[tuple, tuple] = {}
-_cache: dict[tuple, tuple] = {}
-# threads that share a stream share its tables: one call's patch and passes at a time
-_lock = threading.Lock()
+_cache: dict[tuple, _ClipLaunch] = {}
 
 
-def _ws(device, stream: int):
-    """Partial sums and coefficient, one set per (device, stream): calls on different
-    streams may overlap and must not share scratch (calls on one stream are ordered)."""
-    key = (device, stream)
-    ws = _workspace.get(key)
-    if ws is None:
-        if len(_workspace) > 16:
-            # a freed block returns to the pool of the stream it was allocated on, and
-            # any reuse there is ordered after the work already queued on that stream
-            _workspace.clear()
-        ws = _workspace[key] = (
-            torch.zeros(_lib.MAX_NORM_BLOCKS, dtype=torch.float64, device=device),
-            torch.zeros(1, dtype=torch.float32, device=device),
-        )
-    return ws
+class _ClipLaunch(_Launch):
+    """The tables of one list of sizes on one stream, with the scratch its passes write.
+    Calls on different streams may overlap and share neither.  Calls of several threads on
+    one stream share both, so one of them at a time points the tables at its gradients and
+    launches its passes (`lock`)."""
+
+    __slots__ = ("lock", "partials", "coef")
+
+    def __init__(self, rows: np.ndarray, device: torch.device):
+        super().__init__(rows, _CHUNK, device, tables=True)
+        self.lock = threading.Lock()
+        self.partials = torch.zeros(_lib.MAX_NORM_BLOCKS, dtype=torch.float64, device=device)
+        self.coef = torch.zeros(1, dtype=torch.float32, device=device)
 
 
-def _tables(grads, device, stream: int):
-    """The tables of one gradient list.  The chunk table depends on the sizes only and is
-    cached by them, per stream (so the tables are allocated on the stream whose launches
-    read them, and a replaced or dropped table returns to that stream's pool, ordered
-    after those launches); when the gradients moved (zero_grad freed them and backward
-    allocated them elsewhere) only the rows are rewritten."""
-    from .optimizer import _ROW_DTYPE, _Launch
+def _tables(grads, device, stream: int) -> _ClipLaunch:
+    """The tables for gradients of these sizes, cached per stream (so that they are allocated
+    on the stream whose launches read them, and a replaced or dropped table returns to that
+    stream's pool, ordered after those launches).  Cached tables may point at another call's
+    gradients of the same sizes: _run moves them."""
     rows = np.zeros(len(grads), dtype=_ROW_DTYPE)
     ptrs = np.array([g.data_ptr() for g in grads], dtype=np.uint64)
     # Only the gradient pointer is read by the norm and scale kernels.
@@ -61,14 +55,11 @@ def _tables(grads, device, stream: int):
     rows = rows[rows["numel"] > 0]
     key = (device, stream, rows["numel"].tobytes())
     launch = _cache.get(key)
-    if launch is not None:
-        if not np.array_equal(launch.host_rows["grad"], rows["grad"]):
-            launch.set_rows(rows, device)
-        return launch
-    launch = _Launch(rows, _CHUNK, device, tables=True)
-    if len(_cache) > 8:
-        _cache.clear()
-    _cache[key] = launch
+    if launch is None:
+        launch = _ClipLaunch(rows, device)
+        if len(_cache) > 8:
+            _cache.clear()
+        _cache[key] = launch
     return launch
 
 
@@ -89,30 +80,28 @@ def _move(launch, ptrs: bytes, device) -> None:
         launch.rows.data_ptr(), launch.n_rows, len(idx), idx.ctypes.data, new.ctypes.data,
         vec.ctypes.data, torch._C._cuda_getCurrentRawStream(device.index))
     if code != _lib.OK:
-        _cache.clear()      # the device table may hold part of the patch
+        launch.host_rows["grad"] = 0    # the device table may hold part of the patch
     _lib.check(code, "mi_adamw_set_grads")
     launch.host_rows = rows
 
 
-def _run(launch, ptrs: bytes | None, device, stream: int, max_norm: float, norm_type: float,
+def _run(launch, ptrs: bytes, device, stream: int, max_norm: float, norm_type: float,
          error_if_nonfinite: bool) -> torch.Tensor:
-    """The norm and scale passes over a launch's tables; `ptrs`: where the gradients are
-    (None: where the tables say)."""
+    """The norm and scale passes over a launch's tables; `ptrs`: where the gradients are."""
     if torch._C._cuda_getDevice() != device.index:
         with torch.cuda.device(device):
             return _run(launch, ptrs, device, stream, max_norm, norm_type, error_if_nonfinite)
-    with _lock:
+    with launch.lock:
         if torch._C._cuda_isCurrentStreamCapturing():
             launch.recorded = True
-        if ptrs is not None and ptrs != launch.host_rows["grad"].tobytes():
+        if ptrs != launch.host_rows["grad"].tobytes():
             _move(launch, ptrs, device)
         lib = _lib.load()
         norm = torch.empty((), dtype=torch.float32, device=device)
-        partials, coef = _ws(device, stream)
         _lib.check(lib.mi_adamw_grad_norm(
             launch.rows.data_ptr(), launch.chunks.data_ptr(), launch.n_chunks, _CHUNK,
-            float(max_norm), partials.data_ptr(), norm.data_ptr(),
-            coef.data_ptr(), stream), "mi_adamw_grad_norm")
+            float(max_norm), launch.partials.data_ptr(), norm.data_ptr(),
+            launch.coef.data_ptr(), stream), "mi_adamw_grad_norm")
         if error_if_nonfinite and bool(torch.logical_or(norm.isnan(), norm.isinf())):
             raise RuntimeError(
                 f"The total norm of order {float(norm_type)} for gradients from "
@@ -121,7 +110,7 @@ def _run(launch, ptrs: bytes | None, device, stream: int, max_norm: float, norm_
                 "set `error_if_nonfinite=False`")
         _lib.check(lib.mi_adamw_scale_grads(
             launch.rows.data_ptr(), launch.chunks.data_ptr(), launch.n_chunks, _CHUNK,
-            coef.data_ptr(), stream), "mi_adamw_scale_grads")
+            launch.coef.data_ptr(), stream), "mi_adamw_scale_grads")
         return norm
 
 
@@ -158,4 +147,5 @@ def clip_grad_norm_(parameters, max_norm: float, norm_type: float = 2.0,
         launch = _tables(grads, device, stream)
         if launch.n_chunks == 0:
             return torch.zeros((), dtype=torch.float32, device=device)
-    return _run(launch, None, device, stream, max_norm, norm_type, error_if_nonfinite)
+    ptrs = np.array([g.data_ptr() for g in grads if g.numel()], dtype=np.uint64).tobytes()
+    return _run(launch, ptrs, device, stream, max_norm, norm_type, error_if_nonfinite)
