@@ -23,6 +23,9 @@ from .optimizer import _ROW_DTYPE, _Launch
 
 _CHUNK = 4096
 _cache: dict[tuple, _ClipLaunch] = {}
+# what graphs hold the addresses of (_recorded_tables): a graph's end is not announced, so
+# these stay, 64 bytes per gradient and 8 per 4096 elements of each recorded set of tables
+_kept: list = []
 
 
 class _ClipLaunch(_Launch):
@@ -31,10 +34,13 @@ class _ClipLaunch(_Launch):
     one stream share both, so one of them at a time points the tables at its gradients and
     launches its passes (`lock`)."""
 
-    __slots__ = ("lock", "partials", "coef")
+    __slots__ = ("stream", "lock", "partials", "coef", "recorded", "kept")
 
-    def __init__(self, rows: np.ndarray, device: torch.device):
+    def __init__(self, rows: np.ndarray, device: torch.device, stream: int):
         super().__init__(rows, _CHUNK, device, tables=True)
+        self.stream = stream
+        self.recorded = False       # a graph reads the rows, which then never change
+        self.kept = None            # the rows that _kept holds
         self.lock = threading.Lock()
         self.partials = torch.zeros(_lib.MAX_NORM_BLOCKS, dtype=torch.float64, device=device)
         self.coef = torch.zeros(1, dtype=torch.float32, device=device)
@@ -55,17 +61,53 @@ def _tables(grads, device, stream: int) -> _ClipLaunch:
     rows = rows[rows["numel"] > 0]
     key = (device, stream, rows["numel"].tobytes())
     launch = _cache.get(key)
+    if launch is None and device.type == "cuda" and torch.cuda.is_current_stream_capturing():
+        # another stream's tables serve (_recorded_tables); an upload cannot be recorded
+        for (dev, _, numels), other in list(_cache.items()):
+            if dev == device and numels == key[2]:
+                return other
+        raise RuntimeError("mi_adamw.clip_grad_norm_ under graph capture, but no eager call has "
+                           "had gradients of these sizes; run one before capturing")
     if launch is None:
-        launch = _ClipLaunch(rows, device)
+        launch = _ClipLaunch(rows, device, stream)
         if len(_cache) > 8:
             _cache.clear()
         _cache[key] = launch
     return launch
 
 
+def _patch(table: torch.Tensor, n_rows: int, idx: np.ndarray, grads: np.ndarray, device) -> int:
+    """New gradient addresses for the rows idx of a device table, carried there as kernel
+    arguments; the library's code."""
+    grads = np.ascontiguousarray(grads)
+    vec = (grads % 16 == 0).astype(np.uint8)
+    return _lib.load().mi_adamw_set_grads(
+        table.data_ptr(), n_rows, len(idx), idx.ctypes.data, grads.ctypes.data, vec.ctypes.data,
+        torch._C._cuda_getCurrentRawStream(device.index))
+
+
+def _recorded_tables(launch, ptrs: bytes, device, stream: int):
+    """(rows, partial sums, coefficient) for a call that a graph records.  The rows are the
+    launch's where they are this stream's and say where the gradients are; they and the chunk
+    table then stay as they are for good.  Otherwise the graph makes its own, a copy of the
+    launch's with the addresses patched, at each replay: memory of the graph's pool, as the
+    scratch is, which replays and eager calls of the stream would otherwise share."""
+    if launch.kept is not launch.rows:
+        _kept.append((launch.rows, launch.chunks))
+        launch.kept = launch.rows
+    rows = launch.rows
+    if launch.stream == stream and ptrs == launch.host_rows["grad"].tobytes():
+        launch.recorded = True
+    else:
+        rows = rows.clone()
+        _lib.check(_patch(rows, launch.n_rows, np.arange(launch.n_rows, dtype=np.int32),
+                          np.frombuffer(ptrs, dtype=np.uint64), device), "mi_adamw_set_grads")
+    return (rows, torch.empty_like(launch.partials), torch.empty_like(launch.coef))
+
+
 def _move(launch, ptrs: bytes, device) -> None:
     """The gradients lie elsewhere than the launch's table says: the table is patched in
-    place (it belongs to one stream), or replaced if a graph has recorded its address."""
+    place (it belongs to one stream), or replaced if a graph reads it."""
     grads = np.frombuffer(ptrs, dtype=np.uint64)
     rows = launch.host_rows.copy()
     idx = np.flatnonzero(grads != rows["grad"]).astype(np.int32)
@@ -73,12 +115,9 @@ def _move(launch, ptrs: bytes, device) -> None:
     rows["flags"] = np.where(grads % 16 == 0, _lib.T_VEC, 0)
     if launch.recorded:
         launch.set_rows(rows, device)
+        launch.recorded = False
         return
-    new = np.ascontiguousarray(grads[idx])
-    vec = (new % 16 == 0).astype(np.uint8)
-    code = _lib.load().mi_adamw_set_grads(
-        launch.rows.data_ptr(), launch.n_rows, len(idx), idx.ctypes.data, new.ctypes.data,
-        vec.ctypes.data, torch._C._cuda_getCurrentRawStream(device.index))
+    code = _patch(launch.rows, launch.n_rows, idx, grads[idx], device)
     if code != _lib.OK:
         launch.host_rows["grad"] = 0    # the device table may hold part of the patch
     _lib.check(code, "mi_adamw_set_grads")
@@ -93,15 +132,17 @@ def _run(launch, ptrs: bytes, device, stream: int, max_norm: float, norm_type: f
             return _run(launch, ptrs, device, stream, max_norm, norm_type, error_if_nonfinite)
     with launch.lock:
         if torch._C._cuda_isCurrentStreamCapturing():
-            launch.recorded = True
-        if ptrs != launch.host_rows["grad"].tobytes():
-            _move(launch, ptrs, device)
+            rows, partials, coef = _recorded_tables(launch, ptrs, device, stream)
+        else:
+            if ptrs != launch.host_rows["grad"].tobytes():
+                _move(launch, ptrs, device)
+            rows, partials, coef = launch.rows, launch.partials, launch.coef
         lib = _lib.load()
         norm = torch.empty((), dtype=torch.float32, device=device)
         _lib.check(lib.mi_adamw_grad_norm(
-            launch.rows.data_ptr(), launch.chunks.data_ptr(), launch.n_chunks, _CHUNK,
-            float(max_norm), launch.partials.data_ptr(), norm.data_ptr(),
-            launch.coef.data_ptr(), stream), "mi_adamw_grad_norm")
+            rows.data_ptr(), launch.chunks.data_ptr(), launch.n_chunks, _CHUNK,
+            float(max_norm), partials.data_ptr(), norm.data_ptr(),
+            coef.data_ptr(), stream), "mi_adamw_grad_norm")
         if error_if_nonfinite and bool(torch.logical_or(norm.isnan(), norm.isinf())):
             raise RuntimeError(
                 f"The total norm of order {float(norm_type)} for gradients from "
@@ -109,8 +150,8 @@ def _run(launch, ptrs: bytes, device, stream: int, max_norm: float, norm_type: f
                 "this error and scale the gradients by the non-finite norm anyway, "
                 "set `error_if_nonfinite=False`")
         _lib.check(lib.mi_adamw_scale_grads(
-            launch.rows.data_ptr(), launch.chunks.data_ptr(), launch.n_chunks, _CHUNK,
-            launch.coef.data_ptr(), stream), "mi_adamw_scale_grads")
+            rows.data_ptr(), launch.chunks.data_ptr(), launch.n_chunks, _CHUNK,
+            coef.data_ptr(), stream), "mi_adamw_scale_grads")
         return norm
 
 

@@ -205,7 +205,7 @@ class _Launch:
     """Device-resident tensor and chunk tables for one kernel launch."""
 
     __slots__ = ("rows", "chunks", "n_chunks", "n_rows", "host_rows", "tables", "src", "rest",
-                 "step_index", "row_scalars", "recorded")
+                 "step_index", "row_scalars")
 
     def __init__(self, rows: np.ndarray, chunk_elems: int, device: torch.device,
                  tables: bool = False, src: np.ndarray | None = None,
@@ -221,7 +221,6 @@ class _Launch:
                             torch.empty(self.n_rows * _lib.ROW_SCALAR_BYTES, dtype=torch.uint8,
                                         device=device))
         self.host_rows = rows.copy()
-        self.recorded = False       # a graph holds the tables' addresses (clip_grad_norm_)
         self.tables = tables or len(rows) != 1
         # src[i]: the entry whose gradient row i points at (-1: a flat group row, whose
         # gradient buffer never moves); rest[i]: row i's other pointers are aligned
