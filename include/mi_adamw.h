@@ -320,7 +320,9 @@ int mi_adamw_widen_bf16(const mi_adamw_tensor *d_tensors, const mi_adamw_chunk *
  * mi_adamw_tensor.hyper.  d_grad_scale: device fp32 scalar, read with
  * MI_ADAMW_F_CLIP (normally d_coef of mi_adamw_grad_norm on the same stream).
  * state_dtype: MI_ADAMW_STATE_*.  flags: MI_ADAMW_F_*.
- * max_blocks: upper bound on workgroups (0 = one per chunk). */
+ * max_blocks: upper bound on the lanes launched, in units of 1024 (0 = none): the launch
+ * has one workgroup, of 256 or 1024 lanes, per tile of a chunk, and a bounded one's
+ * workgroups take several tiles each. */
 int mi_adamw_step(const mi_adamw_tensor *d_tensors, const mi_adamw_chunk *d_chunks,
                   int64_t n_chunks, int64_t chunk_elems, const mi_adamw_hyper *hypers,
                   int32_t n_hyper, const float *d_grad_scale, int32_t state_dtype,

@@ -48,6 +48,7 @@
 
 #include "mi_adamw.h"
 #include "fp32_math.h"   // bf16x2_bits, bf16_bits, div_by_recip
+#include "items.h"       // Items, item_order, grids
 
 namespace {
 
@@ -863,42 +864,6 @@ __global__ __launch_bounds__(kNormThreads) void mi_adamw_sumsq_reduce_kernel(
 }
 
 // ---------------------------------------------------------------------------
-// Work items of the streaming passes (update, scale, widen): one tile of a chunk each.
-
-// The item that workgroup index w takes: in every full group of 8 runs of kRun items, XCD
-// w % 8 gets one contiguous run, another one from group to group (a fixed one leaves some
-// placements of the update's buffers 3% slower).
-template <int kRun>
-__device__ __forceinline__ int64_t item_order(int64_t w, int64_t n_items) {
-    static_assert((kRun & (kRun - 1)) == 0, "masks and shifts below");
-    constexpr int64_t kGroup = 8 * kRun;
-    const int64_t base = w & ~(kGroup - 1);
-    if (base + kGroup > n_items) return w;
-    const int64_t r = w - base;
-    return base + ((r ^ (w >> __builtin_ctzll(kGroup))) & 7) * kRun + (r >> 3);
-}
-
-// The items of a launch: chunks of chunk_elems elements, `tiles` tiles each.
-struct Items {
-    int64_t n;
-    int64_t chunk_elems;
-    int32_t tiles;
-    int32_t shift;    // log2(tiles), or -1
-    // Item `it`: its chunk's tensor and row, and the tile's elements.  False past the end of
-    // the tensor's last, shorter chunk.
-    template <int kTile, class Src>
-    __device__ __forceinline__ bool get(const Src& src, int64_t it, mi_adamw_tensor& t,
-                                        int64_t& begin, int64_t& end, int32_t& row) const {
-        const int64_t c = shift >= 0 ? it >> shift : it / tiles;
-        src.get(c, chunk_elems, t, begin, end, row);
-        begin += (it - c * tiles) * kTile;
-        if (begin >= end) return false;
-        if (end > begin + kTile) end = begin + kTile;
-        return true;
-    }
-};
-
-// ---------------------------------------------------------------------------
 // Pass 2: the AdamW update.
 //
 // A work item is one tile of a chunk, kThreads * 4 elements, one dwordx4 group per lane:
@@ -1215,21 +1180,6 @@ int launch_status() {
     return e == hipSuccess ? MI_ADAMW_OK : static_cast<int>(e);
 }
 
-unsigned grid_for(int64_t n_chunks, int32_t max_blocks, int threads) {
-    int64_t g = n_chunks;
-    if (max_blocks > 0 && g > max_blocks) g = max_blocks;
-    if (g > 0x7fffffff / threads) g = 0x7fffffff / threads;
-    return static_cast<unsigned>(g);
-}
-
-// The tiles of n_chunks chunks (chunk sizes are multiples of kChunkQuantum, of which every
-// tile size is a divisor).
-Items items_of(int64_t n_chunks, int64_t chunk_elems, int tile) {
-    const int32_t tiles = static_cast<int32_t>(chunk_elems / tile);
-    const int32_t shift = (tiles & (tiles - 1)) == 0 ? __builtin_ctz(tiles) : -1;
-    return Items{n_chunks * tiles, chunk_elems, tiles, shift};
-}
-
 bool aligned(const void* p, uintptr_t a) { return (reinterpret_cast<uintptr_t>(p) & (a - 1)) == 0; }
 
 bool finite(float x) { return x - x == 0.0f; }
@@ -1305,7 +1255,7 @@ int launch_update_k(const Src& src, int64_t n_chunks, int64_t chunk_elems, const
     constexpr int kThreads = update_threads<HS>();
     const Items items = items_of(n_chunks, chunk_elems, kThreads * kVec);
     hipLaunchKernelGGL((mi_adamw_update_kernel<Src, HS, StateT, kClip, kCopy, kWriteGrad, kAms>),
-                       dim3(grid_for(items.n, max_blocks, kThreads)), dim3(kThreads), 0, s, src,
+                       dim3(update_grid(items.n, max_blocks, kThreads)), dim3(kThreads), 0, s, src,
                        items, hs, scale, pre);
     return launch_status();
 }
@@ -1703,8 +1653,8 @@ int mi_adamw_widen_bf16(const mi_adamw_tensor* d_tensors, const mi_adamw_chunk* 
         return MI_ADAMW_E_INVALID;
     TableSource src{d_tensors, d_chunks};
     const Items items = items_of(n_chunks, chunk_elems, kScaleTile);
-    hipLaunchKernelGGL(mi_adamw_widen_kernel, dim3(grid_for(items.n, 0, kScaleThreads)), dim3(kScaleThreads), 0,
-                       static_cast<hipStream_t>(stream), src, items);
+    hipLaunchKernelGGL(mi_adamw_widen_kernel, dim3(grid_for(items.n, 0, kScaleThreads)),
+                       dim3(kScaleThreads), 0, static_cast<hipStream_t>(stream), src, items);
     return launch_status();
 }
 
