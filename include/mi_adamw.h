@@ -42,7 +42,7 @@
 extern "C" {
 #endif
 
-#define MI_ADAMW_ABI_VERSION 9
+#define MI_ADAMW_ABI_VERSION 10
 #define MI_ADAMW_MAX_HYPER 16      /* hyperparameter sets per launch */
 #define MI_ADAMW_MAX_NORM_BLOCKS 4096 /* partial sums per grad-norm launch */
 

@@ -25,7 +25,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_DIR = os.environ.get("MI_ADAMW_LIB_DIR") or HERE
 LIB_PATH = os.path.join(LIB_DIR, "libmi_adamw.so")
 
-ABI_VERSION = 9
+ABI_VERSION = 10
 MAX_HYPER = 16
 MAX_NORM_BLOCKS = 4096
 NOALLOC_SCRATCH_BYTES = 4096

@@ -1472,7 +1472,7 @@ int scratch_on(hipStream_t s, double** out) {
 extern "C" {
 
 const char* mi_adamw_version(void) {
-    return "mi_adamw 9 gfx950 fused clip+adamw (fp32/bf16 state, bf16 copy, amsgrad, flat, "
+    return "mi_adamw 10 gfx950 fused clip+adamw (fp32/bf16 state, bf16 copy, amsgrad, flat, "
            "capturable, fused=True chain, bf16 widen, memory probe, no-alloc norm, range norm, "
            "grad prescale, grad patch)";
 }

@@ -19,7 +19,10 @@
  *                   - torch's fused=True chain: a flat range with the clip, then
  *                     tables with two sets (one without weight decay, with
  *                     maximize), then tables at device step counts with a device
- *                     lr: bit-exact.
+ *                     lr: bit-exact;
+ *                   - the clip through a norm block, folded into the update, finished
+ *                     before it, and deferred to the capturable chain's first launch
+ *                     with the step counts: the bits of the separate launches.
  *
  * The per-step scalars are computed here as the header documents (float64 on
  * the host, as torch/optim/adam.py:529-536 does, then cast to fp32), with
@@ -266,6 +269,40 @@ static int cpu_checks(void)
                                          NULL) == MI_ADAMW_E_ALIGN, "misaligned fused flat range");
     CHECK(mi_adamw_step_flat_fused_chain(&t, NULL, NULL, 1.0f, 4096, MI_ADAMW_STATE_F32, 0, 0,
                                          NULL) == MI_ADAMW_E_INVALID, "fused flat without a set");
+    /* the norm block and the flags that go with it */
+    mi_adamw_norm_block *fake_b = (mi_adamw_norm_block *)(uintptr_t)4096;
+    mi_adamw_norm_block *odd_b = (mi_adamw_norm_block *)(uintptr_t)4100;
+    CHECK(sizeof(mi_adamw_norm_block) == MI_ADAMW_NORM_BLOCK_BYTES, "norm block size");
+    CHECK(mi_adamw_grad_norm_block(NULL, fake, 1, 4096, 1.0f, 1.0f, 0, fake_b, fake_f, NULL) ==
+              MI_ADAMW_E_INVALID, "norm block without tables");
+    CHECK(mi_adamw_grad_norm_block(fake, fake, 1, 4096, 1.0f, 1.0f, 0, NULL, fake_f, NULL) ==
+              MI_ADAMW_E_INVALID, "norm block without a block");
+    CHECK(mi_adamw_grad_norm_block(fake, fake, 1, 4096, 1.0f, 1.0f, 0, fake_b, NULL, NULL) ==
+              MI_ADAMW_E_INVALID, "norm block without a norm");
+    CHECK(mi_adamw_grad_norm_block(fake, fake, 1, 4096, 1.0f, 1.0f, 0, odd_b, fake_f, NULL) ==
+              MI_ADAMW_E_INVALID, "misaligned norm block");
+    CHECK(mi_adamw_grad_norm_block(fake, fake, 1, 4096, NAN, 1.0f, 1, fake_b, fake_f, NULL) ==
+              MI_ADAMW_E_INVALID, "norm block with a NaN pre-scale");
+    CHECK(mi_adamw_grad_norm_block(fake, fake, 1, 1000, 1.0f, 1.0f, 0, fake_b, fake_f, NULL) ==
+              MI_ADAMW_E_INVALID, "norm block chunk size");
+    CHECK(mi_adamw_grad_norm_block_flat(fake_f, 0, 4096, 1.0f, 1.0f, fake_b, fake_f, NULL) ==
+              MI_ADAMW_E_INVALID, "norm block of nothing");
+    CHECK(mi_adamw_grad_norm_block_flat(fake_f, 10, 4096, 1.0f, 1.0f, odd_b, fake_f, NULL) ==
+              MI_ADAMW_E_INVALID, "misaligned flat norm block");
+    CHECK(mi_adamw_step(fake, fake, 1, 4096, h, 1, fake_f, 0, MI_ADAMW_F_NORM_BLOCK, 0, NULL) ==
+              MI_ADAMW_E_INVALID, "a norm block without the clip");
+    CHECK(mi_adamw_step(fake, fake, 1, 4096, h, 1, (const float *)odd_b, 0,
+                        MI_ADAMW_F_CLIP | MI_ADAMW_F_NORM_BLOCK, 0, NULL) == MI_ADAMW_E_INVALID,
+          "step with a misaligned norm block");
+    CHECK(mi_adamw_step(fake, fake, 1, 4096, h, 1, NULL, 0, MI_ADAMW_F_ADVANCE, 0, NULL) ==
+              MI_ADAMW_E_INVALID, "advance without device step counts");
+    CHECK(mi_adamw_step_capturable(fake, fake, 1, 4096, &ch, 1, fake, fake, NULL, 0,
+                                   MI_ADAMW_F_ADVANCE, 0, NULL) == MI_ADAMW_E_INVALID,
+          "advance without the launch that forms the rows");
+    CHECK(mi_adamw_step_capturable_rows(fake, 1, fake, 1, 4096, &ch, 1, fake, fake,
+                                        (void *)(uintptr_t)4096, (const float *)odd_b, 0,
+                                        MI_ADAMW_F_CLIP | MI_ADAMW_F_NORM_BLOCK, 0, NULL) ==
+              MI_ADAMW_E_INVALID, "rows with a misaligned norm block");
     printf("abi_check cpu: ok (%s)\n", mi_adamw_version());
     return 0;
 }
@@ -868,6 +905,121 @@ static void fused_case(void)
            "and lr (both entry points): bit-exact\n");
 }
 
+/* The clip through a norm block against the same step with the norm pass, its finalize and
+ * the step counts apart: the norm's, the parameters' and the moments' bits.  `big`: a set whose
+ * norm is finished before the update.  capt: the capturable chain, deferred and advancing. */
+static void norm_block_case(int big, int capt)
+{
+    enum { NT = 3 };
+    const int64_t numel[NT] = {3, 5000, big ? (1 << 20) + 7 : 4099};
+    mi_adamw_tensor rows[2][NT];
+    memset(rows, 0, sizeof rows);
+    for (int k = 0; k < NT; ++k) {
+        const int64_t n = numel[k];
+        float *x = malloc(n * 4);
+        CHECK(x, "host allocation");
+        for (int f = 0; f < 4; ++f) {
+            fill(x, n, f == 1 ? 1e-1f : 1e-3f, f == 3);
+            for (int side = 0; side < 2; ++side) {
+                void *d = dev_copy(x, n * 4);
+                if (f == 0) rows[side][k].param = d;
+                if (f == 1) rows[side][k].grad = d;
+                if (f == 2) rows[side][k].exp_avg = d;
+                if (f == 3) rows[side][k].exp_avg_sq = d;
+            }
+        }
+        free(x);
+        for (int side = 0; side < 2; ++side) {
+            rows[side][k].numel = n;
+            rows[side][k].flags = MI_ADAMW_T_VEC;
+        }
+    }
+    const int64_t nc = mi_adamw_build_chunks(numel, NT, 4096, NULL, 0);
+    mi_adamw_chunk *chunks = malloc(nc * sizeof *chunks);
+    CHECK(chunks && mi_adamw_build_chunks(numel, NT, 4096, chunks, nc) == nc, "chunks");
+    void *d_chunks = dev_copy(chunks, nc * sizeof *chunks);
+    void *d_rows[2] = {dev_copy(rows[0], sizeof rows[0]), dev_copy(rows[1], sizeof rows[1])};
+    const float counts[2][NT] = {{1001.0f, 8.0f, 3.0f}, {1000.0f, 7.0f, 2.0f}};
+    const int32_t index[NT] = {2, 0, 1};
+    void *d_steps[2] = {dev_copy(counts[0], sizeof counts[0]),
+                        dev_copy(counts[1], sizeof counts[1])};
+    void *d_index = dev_copy(index, sizeof index);
+    void *scalars_buf = NULL;
+    double *dpart = NULL;
+    float *dnorm = NULL, *dcoef = NULL;
+    mi_adamw_norm_block *block = NULL;
+    HIP(hipMalloc(&scalars_buf, NT * MI_ADAMW_ROW_SCALAR_BYTES));
+    HIP(hipMalloc((void **)&dpart, MI_ADAMW_MAX_NORM_BLOCKS * sizeof(double)));
+    HIP(hipMalloc((void **)&dnorm, 2 * sizeof(float)));
+    HIP(hipMalloc((void **)&dcoef, sizeof(float)));
+    HIP(hipMalloc((void **)&block, MI_ADAMW_NORM_BLOCK_BYTES));
+    mi_adamw_hyper h;
+    oracle_hyper oh;
+    scalars(3e-4, 0.9, 0.95, 1e-8, 0.1, 1001.0, 0, &h, &oh);
+    mi_adamw_capt_hyper ch;
+    memset(&ch, 0, sizeof ch);
+    ch.beta1 = 0.9f;
+    ch.beta2 = 0.95f;
+    ch.lerp_w = 1.0f - 0.9f;
+    ch.one_minus_beta2 = 1.0f - 0.95f;
+    ch.eps = 1e-8f;
+    ch.grad_sign = 1.0f;
+    ch.lr_mode = MI_ADAMW_LR_FLOAT;
+    ch.lr = 1e-3f;
+    ch.wd_factor = 1.0f - 1e-4f;
+    for (int side = 0; side < 2; ++side) {
+        const float *scale = side ? (const float *)block : dcoef;
+        const int32_t flags = MI_ADAMW_F_CLIP | (side ? MI_ADAMW_F_NORM_BLOCK : 0);
+        int rc = side ? mi_adamw_grad_norm_block(d_rows[1], d_chunks, nc, 4096, 1.0f, 0.5f, capt,
+                                                 block, dnorm + 1, NULL)
+                      : mi_adamw_grad_norm(d_rows[0], d_chunks, nc, 4096, 0.5f, dpart, dnorm,
+                                           dcoef, NULL);
+        CHECK(rc == 0, "norm: %s", mi_adamw_strerror(rc));
+        rc = capt ? mi_adamw_step_capturable_rows(d_rows[side], NT, d_chunks, nc, 4096, &ch, 1,
+                                                  d_steps[side], d_index, scalars_buf, scale,
+                                                  MI_ADAMW_STATE_F32,
+                                                  flags | (side ? MI_ADAMW_F_ADVANCE : 0), 0, NULL)
+                  : mi_adamw_step(d_rows[side], d_chunks, nc, 4096, &h, 1, scale,
+                                  MI_ADAMW_STATE_F32, flags, 0, NULL);
+        CHECK(rc == 0, "step: %s", mi_adamw_strerror(rc));
+    }
+    HIP(hipDeviceSynchronize());
+    float norm[2], after[2][NT];
+    back(norm, dnorm, sizeof norm);
+    CHECK(memcmp(&norm[0], &norm[1], 4) == 0 && norm[0] > 0.5f, "norms %.9g and %.9g", norm[0],
+          norm[1]);
+    back(after[0], d_steps[0], sizeof after[0]);
+    back(after[1], d_steps[1], sizeof after[1]);
+    CHECK(!capt || memcmp(after[0], after[1], sizeof after[0]) == 0, "step counts");
+    for (int k = 0; k < NT; ++k) {
+        float *a = malloc(numel[k] * 4), *b = malloc(numel[k] * 4);
+        CHECK(a && b, "host allocation");
+        for (int f = 0; f < 3; ++f) {
+            back(a, f == 0 ? (void *)rows[0][k].param : f == 1 ? rows[0][k].exp_avg
+                                                               : rows[0][k].exp_avg_sq,
+                 numel[k] * 4);
+            back(b, f == 0 ? (void *)rows[1][k].param : f == 1 ? rows[1][k].exp_avg
+                                                               : rows[1][k].exp_avg_sq,
+                 numel[k] * 4);
+            CHECK(memcmp(a, b, numel[k] * 4) == 0, "norm block, tensor %d, field %d", k, f);
+        }
+        free(a);
+        free(b);
+        for (int side = 0; side < 2; ++side) {
+            HIP(hipFree(rows[side][k].param)); HIP(hipFree(rows[side][k].grad));
+            HIP(hipFree(rows[side][k].exp_avg)); HIP(hipFree(rows[side][k].exp_avg_sq));
+        }
+    }
+    for (int side = 0; side < 2; ++side) {
+        HIP(hipFree(d_rows[side])); HIP(hipFree(d_steps[side]));
+    }
+    HIP(hipFree(d_chunks)); HIP(hipFree(d_index)); HIP(hipFree(scalars_buf));
+    HIP(hipFree(dpart)); HIP(hipFree(dnorm)); HIP(hipFree(dcoef)); HIP(hipFree(block));
+    free(chunks);
+    printf("abi_check gpu: norm block, %s%s: the bits of the separate launches\n",
+           capt ? "capturable, advancing" : "default chain", big ? ", large set" : "");
+}
+
 static int gpu_checks(void)
 {
     int count = 0;
@@ -881,6 +1033,7 @@ static int gpu_checks(void)
     split_case(3000000 + 96, 3);
     set_grads_case();
     fused_case();
+    for (int k = 0; k < 4; ++k) norm_block_case(k & 1, k >> 1);
     printf("abi_check gpu: ok (%s)\n", mi_adamw_version());
     return 0;
 }
