@@ -74,6 +74,11 @@ extern "C" {
                                           first (every row then has an index of its own), in
                                           place of a launch that increments them (adam.py:414) */
 
+#define MI_ADAMW_F_TILES (1 << 6)      /* tables: d_chunks and n_chunks are the tiles of
+                                          mi_adamw_build_tiles, not chunks of chunk_elems.
+                                          Not with mi_adamw_step_capturable, whose
+                                          workgroups take 4096 elements */
+
 /* mi_adamw_tensor.flags */
 #define MI_ADAMW_T_VEC (1 << 0) /* promises fp32 pointers 16-byte aligned and bf16 pointers
                                    8-byte aligned (the flat entry points check it); the
@@ -189,6 +194,15 @@ const char *mi_adamw_strerror(int code);
  * out == NULL only counts. */
 int64_t mi_adamw_build_chunks(const int64_t *numels, int32_t n_tensors, int64_t chunk_elems,
                               mi_adamw_chunk *out, int64_t cap);
+
+/* The same for tiles of MI_ADAMW_TILE_ELEMS elements, which an update or a probe takes with
+ * MI_ADAMW_F_TILES.  Without it the launch has chunk_elems / 1024 workgroups per chunk, and
+ * those past the end of a short tensor cost about half a nanosecond each: worth it where most
+ * chunks are far from full (2,000 tensors of 768 elements 16.7 -> 8.4 us; at chunk_elems
+ * 65536 74, at 2^20 1009). */
+#define MI_ADAMW_TILE_ELEMS 1024
+int64_t mi_adamw_build_tiles(const int64_t *numels, int32_t n_tensors, mi_adamw_chunk *out,
+                             int64_t cap);
 
 /* Global gradient L2 norm and clip coefficient (two launches: the float64
  * sum-of-squares pass over a fixed grid, then a one-workgroup reduction).
@@ -433,8 +447,7 @@ int mi_adamw_step_fused_chain_rows(const mi_adamw_tensor *d_tensors, int32_t n_r
 /* Measurement helper with no counterpart in the reference, for benchmarks that want
  * the memory ceiling of the update on the tensors it actually runs on: the same
  * launch as mi_adamw_step / mi_adamw_step_flat (tables or one flat range, launch
- * shape, access widths, cache hints, software pipelining) with the arithmetic left
- * out.  Every loaded value is stored back unchanged and the bf16 copy is written as
+ * shape, order, access widths, cache hints) with the arithmetic left out.  Every loaded value is stored back unchanged and the bf16 copy is written as
  * the bf16 of its master (equal to what the step leaves there), so the bytes moved
  * are exactly the step's and the tensors keep their values.  MI_ADAMW_F_CLIP is
  * accepted and ignored (the gradient is read either way); the other flags select

@@ -31,6 +31,7 @@ MAX_NORM_BLOCKS = 4096
 NOALLOC_SCRATCH_BYTES = 4096
 NORM_BLOCK_BYTES = 4160   # one mi_adamw_norm_block
 CHUNK_QUANTUM = 4096
+TILE_ELEMS = 1024
 ROW_SCALAR_BYTES = 64   # per table row, mi_adamw_step_capturable_rows
 
 OK = 0
@@ -47,6 +48,7 @@ F_WRITE_GRAD = 1 << 2
 F_AMSGRAD = 1 << 3
 F_NORM_BLOCK = 1 << 4
 F_ADVANCE = 1 << 5
+F_TILES = 1 << 6
 
 T_VEC = 1 << 0
 
@@ -59,6 +61,7 @@ EXPORTS = (
     "mi_adamw_version",
     "mi_adamw_strerror",
     "mi_adamw_build_chunks",
+    "mi_adamw_build_tiles",
     "mi_adamw_grad_norm",
     "mi_adamw_grad_norm_flat",
     "mi_adamw_grad_norm_block",
@@ -169,6 +172,7 @@ _SIGNATURES = {
     "mi_adamw_version": ([], ctypes.c_char_p),
     "mi_adamw_strerror": ([ctypes.c_int], ctypes.c_char_p),
     "mi_adamw_build_chunks": ([_vp, _i32, _i64, _vp, _i64], _i64),
+    "mi_adamw_build_tiles": ([_vp, _i32, _vp, _i64], _i64),
     "mi_adamw_grad_norm": ([_vp, _vp, _i64, _i64, _f32, _vp, _vp, _vp, _vp], ctypes.c_int),
     "mi_adamw_grad_norm_flat": ([_vp, _i64, _i64, _f32, _vp, _vp, _vp, _vp], ctypes.c_int),
     "mi_adamw_grad_norm_block": ([_vp, _vp, _i64, _i64, _f32, _f32, _i32, _vp, _vp, _vp],

@@ -108,6 +108,8 @@ struct Plan {
     mi_adamw_tensor flat_row{};      // the single row of a table-free launch
     mi_adamw_tensor* d_rows = nullptr;
     const mi_adamw_chunk* d_chunks = nullptr;
+    const mi_adamw_chunk* d_items = nullptr;   // the update's: the chunks, or with
+    int64_t n_items = 0;                       // MI_ADAMW_F_TILES in flags the tiles
     uint8_t* host_rows = nullptr;    // the host copy of the rows (64 B each), kept in step
     int64_t n_chunks = 0;
     int32_t n_rows = 0;
@@ -189,7 +191,7 @@ PyObject* py_bind(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
 //   launch:          (tables, d_rows, d_chunks, n_chunks, n_rows, host_rows, flat_row_addr,
 //                     flat_hyper)
 //   options:         (chunk_elems, max_blocks, state_code, flags, clip, max_norm, prescale,
-//                     norm_block, grad_scale, 0, stream, fused_chain)
+//                     norm_block, grad_scale, 0, stream, fused_chain[, d_items, n_items])
 //   keep:            objects to keep alive while the plan exists
 PyObject* plan_new(PyObject* args);
 
@@ -269,11 +271,14 @@ PyObject* plan_new(PyObject* args) {
         long long chunk = 0;
         int max_blocks = 0, state_code = 0, flags = 0, clip = 0, fused_chain = 0;
         float max_norm = 0, prescale = 1;
-        unsigned long long block = 0, scale = 0, unused = 0, stream = 0;
-        if (!PyArg_ParseTuple(opts_t, "LiiipffKKKKp", &chunk, &max_blocks, &state_code, &flags,
+        unsigned long long block = 0, scale = 0, unused = 0, stream = 0, items = 0;
+        long long n_items = 0;
+        if (!PyArg_ParseTuple(opts_t, "LiiipffKKKKp|KL", &chunk, &max_blocks, &state_code, &flags,
                               &clip, &max_norm, &prescale, &block, &scale, &unused, &stream,
-                              &fused_chain))
+                              &fused_chain, &items, &n_items))
             goto fail;
+        pl->d_items = items ? reinterpret_cast<const mi_adamw_chunk*>(items) : pl->d_chunks;
+        pl->n_items = items ? n_items : pl->n_chunks;
         pl->fused_chain = fused_chain;
         pl->chunk_elems = chunk;
         pl->max_blocks = max_blocks;
@@ -501,7 +506,7 @@ PyObject* py_update(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     if (pl->fused_chain) {
         const mi_adamw_fused_hyper* fh = static_cast<const mi_adamw_fused_hyper*>(hv);
         if (pl->tables) {
-            rc = g_api.step_fused_chain(pl->d_rows, pl->d_chunks, pl->n_chunks, pl->chunk_elems,
+            rc = g_api.step_fused_chain(pl->d_rows, pl->d_items, pl->n_items, pl->chunk_elems,
                                         fh, static_cast<int32_t>(nh), nullptr, nullptr,
                                         pl->scale, pl->prescale, pl->state_code, flags,
                                         pl->max_blocks, s);
@@ -515,7 +520,7 @@ PyObject* py_update(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     }
     const mi_adamw_hyper* h = static_cast<const mi_adamw_hyper*>(hv);
     if (pl->tables) {
-        rc = g_api.step_prescaled(pl->d_rows, pl->d_chunks, pl->n_chunks, pl->chunk_elems, h,
+        rc = g_api.step_prescaled(pl->d_rows, pl->d_items, pl->n_items, pl->chunk_elems, h,
                                   static_cast<int32_t>(nh), pl->scale, pl->prescale,
                                   pl->state_code, flags, pl->max_blocks, s);
     } else {

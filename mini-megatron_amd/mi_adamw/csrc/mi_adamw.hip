@@ -44,6 +44,7 @@
 #include <atomic>
 #include <cmath>
 #include <mutex>
+#include <type_traits>
 #include <vector>
 
 #include "mi_adamw.h"
@@ -1175,6 +1176,26 @@ bool chunk_elems_ok(int64_t chunk_elems) {
            chunk_elems <= (int64_t(1) << 30);
 }
 
+// The table of tensors cut every chunk_elems elements (mi_adamw_build_chunks).
+int64_t cut_tensors(const int64_t* numels, int32_t n_tensors, int64_t chunk_elems,
+                    mi_adamw_chunk* out, int64_t cap) {
+    if (!numels || n_tensors < 0) return MI_ADAMW_E_INVALID;
+    int64_t n = 0;
+    for (int32_t t = 0; t < n_tensors; ++t) {
+        if (numels[t] < 0) return MI_ADAMW_E_INVALID;
+        const int64_t k = (numels[t] + chunk_elems - 1) / chunk_elems;
+        if (k > 0x7fffffff) return MI_ADAMW_E_INVALID;
+        for (int64_t i = 0; i < k; ++i, ++n) {
+            if (out) {
+                if (n >= cap) return MI_ADAMW_E_INVALID;
+                out[n].tensor = t;
+                out[n].index = static_cast<int32_t>(i);
+            }
+        }
+    }
+    return n;
+}
+
 int launch_status() {
     hipError_t e = hipGetLastError();
     return e == hipSuccess ? MI_ADAMW_OK : static_cast<int>(e);
@@ -1286,14 +1307,30 @@ int launch_update_cw(const Src& src, int64_t n_chunks, int64_t chunk_elems, cons
     return MI_ADAMW_E_INVALID;
 }
 
+// Whether an update's tables may be the tiles of mi_adamw_build_tiles: one workgroup each.
+template <class Src, class HS>
+constexpr bool takes_tiles() {
+    return std::is_same<Src, TableSource>::value &&
+           update_threads<HS>() * kVec == MI_ADAMW_TILE_ELEMS;
+}
+
+// The chunk size of the table that an update's flags name, without the flag.
+int64_t table_elems(int64_t chunk_elems, int32_t& flags) {
+    const bool tiles = flags & MI_ADAMW_F_TILES;
+    flags &= ~MI_ADAMW_F_TILES;
+    return tiles ? MI_ADAMW_TILE_ELEMS : chunk_elems;
+}
+
 // Whether launch_update takes these arguments.
+template <class Src, class HS>
 bool update_args_ok(int64_t n_chunks, int64_t chunk_elems, const float* scale,
                     int32_t state_dtype, int32_t flags) {
     if (n_chunks <= 0 || !chunk_elems_ok(chunk_elems)) return false;
     if (state_dtype != MI_ADAMW_STATE_F32 && state_dtype != MI_ADAMW_STATE_BF16) return false;
     if (flags & ~(MI_ADAMW_F_CLIP | MI_ADAMW_F_BF16_COPY | MI_ADAMW_F_WRITE_GRAD |
-                  MI_ADAMW_F_AMSGRAD | MI_ADAMW_F_NORM_BLOCK))
+                  MI_ADAMW_F_AMSGRAD | MI_ADAMW_F_NORM_BLOCK | MI_ADAMW_F_TILES))
         return false;
+    if ((flags & MI_ADAMW_F_TILES) && !takes_tiles<Src, HS>()) return false;
     const bool block = flags & MI_ADAMW_F_NORM_BLOCK;
     if ((flags & MI_ADAMW_F_CLIP) ? !scale : block) return false;
     return !block || aligned(scale, 8);
@@ -1303,8 +1340,9 @@ template <class Src, class HS>
 int launch_update(const Src& src, int64_t n_chunks, int64_t chunk_elems, const HS& hs,
                   const float* scale, int32_t state_dtype, int32_t flags, int32_t max_blocks,
                   hipStream_t s, float pre = 1.0f) {
-    if (!update_args_ok(n_chunks, chunk_elems, scale, state_dtype, flags))
+    if (!update_args_ok<Src, HS>(n_chunks, chunk_elems, scale, state_dtype, flags))
         return MI_ADAMW_E_INVALID;
+    chunk_elems = table_elems(chunk_elems, flags);
     const bool clip = flags & MI_ADAMW_F_CLIP, block = flags & MI_ADAMW_F_NORM_BLOCK;
 #define MI_ADAMW_CLIP(S)                                                                       \
     (block  ? launch_update_cw<Src, HS, S, kBlock>(src, n_chunks, chunk_elems, hs, scale, pre, \
@@ -1339,8 +1377,11 @@ int launch_probe(const Src& src, int64_t n_chunks, int64_t chunk_elems, int32_t 
     if (state_dtype != MI_ADAMW_STATE_F32 && state_dtype != MI_ADAMW_STATE_BF16)
         return MI_ADAMW_E_INVALID;
     flags &= ~MI_ADAMW_F_CLIP;
-    if (flags & ~(MI_ADAMW_F_BF16_COPY | MI_ADAMW_F_WRITE_GRAD | MI_ADAMW_F_AMSGRAD))
+    if (flags & ~(MI_ADAMW_F_BF16_COPY | MI_ADAMW_F_WRITE_GRAD | MI_ADAMW_F_AMSGRAD |
+                  MI_ADAMW_F_TILES))
         return MI_ADAMW_E_INVALID;
+    if ((flags & MI_ADAMW_F_TILES) && !takes_tiles<Src, ProbeHyper>()) return MI_ADAMW_E_INVALID;
+    chunk_elems = table_elems(chunk_elems, flags);
     const ProbeHyper hs;
     if (state_dtype == MI_ADAMW_STATE_F32)
         return launch_update_cw<Src, ProbeHyper, float, kNoClip>(src, n_chunks, chunk_elems, hs,
@@ -1489,21 +1530,13 @@ const char* mi_adamw_strerror(int code) {
 
 int64_t mi_adamw_build_chunks(const int64_t* numels, int32_t n_tensors, int64_t chunk_elems,
                               mi_adamw_chunk* out, int64_t cap) {
-    if (!numels || n_tensors < 0 || !chunk_elems_ok(chunk_elems)) return MI_ADAMW_E_INVALID;
-    int64_t n = 0;
-    for (int32_t t = 0; t < n_tensors; ++t) {
-        if (numels[t] < 0) return MI_ADAMW_E_INVALID;
-        const int64_t k = (numels[t] + chunk_elems - 1) / chunk_elems;
-        if (k > 0x7fffffff) return MI_ADAMW_E_INVALID;
-        for (int64_t i = 0; i < k; ++i, ++n) {
-            if (out) {
-                if (n >= cap) return MI_ADAMW_E_INVALID;
-                out[n].tensor = t;
-                out[n].index = static_cast<int32_t>(i);
-            }
-        }
-    }
-    return n;
+    if (!chunk_elems_ok(chunk_elems)) return MI_ADAMW_E_INVALID;
+    return cut_tensors(numels, n_tensors, chunk_elems, out, cap);
+}
+
+int64_t mi_adamw_build_tiles(const int64_t* numels, int32_t n_tensors, mi_adamw_chunk* out,
+                             int64_t cap) {
+    return cut_tensors(numels, n_tensors, MI_ADAMW_TILE_ELEMS, out, cap);
 }
 
 int mi_adamw_grad_norm(const mi_adamw_tensor* d_tensors, const mi_adamw_chunk* d_chunks,
@@ -1732,8 +1765,8 @@ int mi_adamw_step_capturable_rows(const mi_adamw_tensor* d_tensors, int32_t n_ro
     CaptHyper hs;
     if (!d_tensors || n_rows <= 0 || !d_chunks || !d_row_scalars || !aligned(d_row_scalars, 16) ||
         capt_hyper_from(hypers, n_hyper, d_steps, d_step_index, hs) ||
-        !update_args_ok(n_chunks, chunk_elems, d_grad_scale, state_dtype,
-                        flags & ~MI_ADAMW_F_ADVANCE))
+        !update_args_ok<TableSource, CaptRowsHyper>(n_chunks, chunk_elems, d_grad_scale,
+                                                    state_dtype, flags & ~MI_ADAMW_F_ADVANCE))
         return MI_ADAMW_E_INVALID;
     const hipStream_t s = static_cast<hipStream_t>(stream);
     RowScalars* rows = static_cast<RowScalars*>(d_row_scalars);
@@ -1783,8 +1816,8 @@ int mi_adamw_step_fused_chain_rows(const mi_adamw_tensor* d_tensors, int32_t n_r
     if (!d_tensors || n_rows <= 0 || !d_chunks || !hypers || n_hyper <= 0 ||
         n_hyper > MI_ADAMW_MAX_HYPER || !finite(grad_prescale) || !d_steps || !d_step_index ||
         !d_row_scalars || !aligned(d_row_scalars, 16) ||
-        !update_args_ok(n_chunks, chunk_elems, d_grad_scale, state_dtype,
-                        flags & ~MI_ADAMW_F_ADVANCE))
+        !update_args_ok<TableSource, FusedRowsHyper>(n_chunks, chunk_elems, d_grad_scale,
+                                                     state_dtype, flags & ~MI_ADAMW_F_ADVANCE))
         return MI_ADAMW_E_INVALID;
     FusedHyper<true> hs;
     memset(&hs, 0, sizeof(hs));

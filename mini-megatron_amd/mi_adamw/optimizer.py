@@ -201,15 +201,28 @@ def _upload(arr: np.ndarray, device: torch.device) -> torch.Tensor:
     return host.pin_memory().to(device, non_blocking=True)
 
 
+# An update of chunks has a workgroup for each tile of a full one; those of a shorter one's
+# missing tiles start, look their tensor up and end.  Where they are more than a fifth of all
+# and more than one for each CU, the update gets a table of the tiles instead.  Default chain,
+# us, chunks -> tiles:
+#   2000 x 768 elements       17.9 ->  8.0      300 x 768    4.1 -> 3.15     50 x 768  2.8 -> 2.7
+#   2000 x 2500 (a quarter)   26.5 -> 24.0      the same with chunk_elems=65536, 2000 x 768: 74
+#   2000 x 768 + 350 x 65536 (a fifth)  120.0 -> 112.3; a twentieth and less (GPTs of 2M
+#   elements and more): 8.35 -> 8.65 at 2M, 546 -> 542 at 124M, four times the table to build
+_TILE_RULE = 1.25
+_TILE_LEAST = 256
+
+
 class _Launch:
     """Device-resident tensor and chunk tables for one kernel launch."""
 
     __slots__ = ("rows", "chunks", "n_chunks", "n_rows", "host_rows", "tables", "src", "rest",
-                 "step_index", "row_scalars")
+                 "step_index", "row_scalars", "items", "n_items", "item_flag")
 
     def __init__(self, rows: np.ndarray, chunk_elems: int, device: torch.device,
                  tables: bool = False, src: np.ndarray | None = None,
-                 rest: np.ndarray | None = None, step_slots: np.ndarray | None = None):
+                 rest: np.ndarray | None = None, step_slots: np.ndarray | None = None,
+                 update: bool = False):
         lib = _lib.load()
         self.n_rows = len(rows)
         # capturable launches: row i's index into the device step buffer, and the device
@@ -230,7 +243,8 @@ class _Launch:
             # One contiguous range: launched through the flat entry points,
             # which derive chunk bounds arithmetically and need no tables.
             self.n_chunks = -(-int(rows["numel"][0]) // chunk_elems)
-            self.rows = self.chunks = None
+            self.rows = self.chunks = self.items = None
+            self.n_items, self.item_flag = self.n_chunks, 0
             return
         numels = np.ascontiguousarray(rows["numel"], dtype=np.int64)
         n = lib.mi_adamw_build_chunks(numels.ctypes.data, len(numels), chunk_elems, None, 0)
@@ -243,6 +257,18 @@ class _Launch:
         self.n_chunks = int(n)
         self.rows = _upload(self.host_rows, device)
         self.chunks = _upload(chunks, device)
+        # what an update takes: the chunks, or the tiles where most chunks are far from full
+        self.items, self.n_items, self.item_flag = self.chunks, self.n_chunks, 0
+        n_tiles = int((-(-numels // _lib.TILE_ELEMS)).sum())
+        n_groups = self.n_chunks * (chunk_elems // _lib.TILE_ELEMS)
+        if update and n_groups > max(_TILE_RULE * n_tiles, n_tiles + _TILE_LEAST):
+            tiles = np.empty(n_tiles * 2, dtype=np.int32)
+            n = lib.mi_adamw_build_tiles(numels.ctypes.data, len(numels), tiles.ctypes.data,
+                                         n_tiles)
+            if n != n_tiles:
+                raise _lib.MiAdamwError("mi_adamw_build_tiles: inconsistent tile count")
+            self.items, self.n_items = _upload(tiles, device), n_tiles
+            self.item_flag = _lib.F_TILES
 
     def set_rows(self, rows: np.ndarray, device: torch.device) -> bool:
         """New pointers for the same tensors (the gradients moved): replace the rows,
@@ -992,6 +1018,7 @@ class FusedAdamW(Optimizer):
                 rest[i] = bool(launch.rest[r])
         hyper_steps = np.zeros(len(hyper_group), dtype=np.float64)
         flat_row = None if launch.tables else self._row_struct(launch)
+        flags |= launch.item_flag
         if ams:
             flags |= _lib.F_AMSGRAD
         clip = self.max_grad_norm is not None
@@ -1011,9 +1038,10 @@ class FusedAdamW(Optimizer):
                  0 if launch.tables else int(launch.host_rows[0]["hyper"])),
                 (int(self.chunk_elems), int(self.max_blocks), int(state_code), int(flags), clip,
                  float(self.max_grad_norm or 0.0), float(self.grad_prescale),
-                 block.data_ptr(), block.data_ptr(), 0, int(stream), bool(fused)),
-                (launch.rows, launch.chunks, launch.host_rows, self._steps, hyper_steps,
-                 block))
+                 block.data_ptr(), block.data_ptr(), 0, int(stream), bool(fused),
+                 0 if launch.items is None else launch.items.data_ptr(), int(launch.n_items)),
+                (launch.rows, launch.chunks, launch.items, launch.host_rows, self._steps,
+                 hyper_steps, block))
         except (TypeError, ValueError):
             return None     # a state entry the plan cannot check (not a tensor): general path
         fast = _Fast()
@@ -1125,9 +1153,9 @@ class FusedAdamW(Optimizer):
             rows, src, rest = self._tensor_rows(entries, hyper_idx, ams)
             slots = np.asarray([entries[i][0].slot for i in src], dtype=np.int32)
             return _Launch(rows, self.chunk_elems, device, tables=True, src=src, rest=rest,
-                           step_slots=slots)
+                           step_slots=slots, update=True)
         rows, src, rest = self._rows(entries, hyper_idx, ams)
-        return _Launch(rows, self.chunk_elems, device, src=src, rest=rest)
+        return _Launch(rows, self.chunk_elems, device, src=src, rest=rest, update=True)
 
     def _flat_rows(self, entries, hyper_idx, ams):
         """One row per param group whose every param steps with one hyper set."""
@@ -1318,15 +1346,15 @@ class FusedAdamW(Optimizer):
         for launch, (_, _, hs, (ams, fused), _) in zip(launches, parts):
             if launch.n_chunks == 0:
                 continue
-            lflags = flags | advance | (_lib.F_AMSGRAD if ams else 0)
+            lflags = flags | advance | launch.item_flag | (_lib.F_AMSGRAD if ams else 0)
             if fused:
                 self._launch_fused_chain(launch, hs, norm_block, state_code, lflags, stream)
                 continue
             if self.capturable:
                 carr = (_lib.CaptHyper * len(hs))(*hs)
                 _lib.check(lib.mi_adamw_step_capturable_rows(
-                    launch.rows.data_ptr(), launch.n_rows, launch.chunks.data_ptr(),
-                    launch.n_chunks, self.chunk_elems, carr, len(hs), self._steps.data_ptr(),
+                    launch.rows.data_ptr(), launch.n_rows, launch.items.data_ptr(),
+                    launch.n_items, self.chunk_elems, carr, len(hs), self._steps.data_ptr(),
                     launch.step_index.data_ptr(), launch.row_scalars.data_ptr(),
                     norm_block.data_ptr(), state_code, lflags, self.max_blocks, stream),
                     "mi_adamw_step_capturable_rows")
@@ -1348,12 +1376,12 @@ class FusedAdamW(Optimizer):
                 continue
             if pre != 1.0:
                 _lib.check(lib.mi_adamw_step_prescaled(
-                    launch.rows.data_ptr(), launch.chunks.data_ptr(), launch.n_chunks,
+                    launch.rows.data_ptr(), launch.items.data_ptr(), launch.n_items,
                     self.chunk_elems, harr, len(hs), norm_block.data_ptr(), pre, state_code, lflags,
                     self.max_blocks, stream), "mi_adamw_step_prescaled")
                 continue
             _lib.check(lib.mi_adamw_step(
-                launch.rows.data_ptr(), launch.chunks.data_ptr(), launch.n_chunks,
+                launch.rows.data_ptr(), launch.items.data_ptr(), launch.n_items,
                 self.chunk_elems, harr, len(hs), norm_block.data_ptr(), state_code, lflags,
                 self.max_blocks, stream), "mi_adamw_step")
         _record(ev, 2)
@@ -1380,7 +1408,7 @@ class FusedAdamW(Optimizer):
         if self.capturable:
             # device step counts: the per-step values formed once per row before the update
             _lib.check(lib.mi_adamw_step_fused_chain_rows(
-                launch.rows.data_ptr(), launch.n_rows, launch.chunks.data_ptr(), launch.n_chunks,
+                launch.rows.data_ptr(), launch.n_rows, launch.items.data_ptr(), launch.n_items,
                 self.chunk_elems, farr, len(hs), self._steps.data_ptr(),
                 launch.step_index.data_ptr(), launch.row_scalars.data_ptr(), block.data_ptr(),
                 pre, state_code, flags, self.max_blocks, stream),
@@ -1388,6 +1416,6 @@ class FusedAdamW(Optimizer):
             return
         # host step counts (hs[i].step): no step buffer
         _lib.check(lib.mi_adamw_step_fused_chain(
-            launch.rows.data_ptr(), launch.chunks.data_ptr(), launch.n_chunks, self.chunk_elems,
+            launch.rows.data_ptr(), launch.items.data_ptr(), launch.n_items, self.chunk_elems,
             farr, len(hs), None, None, block.data_ptr(), pre, state_code, flags, self.max_blocks,
             stream), "mi_adamw_step_fused_chain")

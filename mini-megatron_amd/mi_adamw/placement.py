@@ -173,7 +173,8 @@ class _TableStreams(_Streams):
         arr = np.zeros(len(rows), dtype=self._row_dtype)
         for i, r in enumerate(rows):
             arr[i] = r
-        return self._launch_cls(arr, self.opt.chunk_elems, self.device, tables=True)
+        return self._launch_cls(arr, self.opt.chunk_elems, self.device, tables=True,
+                                update=True)
 
     def twin(self, cand, launches):
         opt, lib = self.opt, _lib.load()
@@ -183,9 +184,10 @@ class _TableStreams(_Streams):
         flags = _twin_flags(opt)
 
         def run():
-            _lib.check(lib.mi_adamw_probe(launch.rows.data_ptr(), launch.chunks.data_ptr(),
-                                          launch.n_chunks, opt.chunk_elems, state, flags,
-                                          opt.max_blocks, stream), "mi_adamw_probe")
+            _lib.check(lib.mi_adamw_probe(launch.rows.data_ptr(), launch.items.data_ptr(),
+                                          launch.n_items, opt.chunk_elems, state,
+                                          flags | launch.item_flag, opt.max_blocks, stream),
+                       "mi_adamw_probe")
         return _timed(run, launches)
 
     def adopt(self, cand):

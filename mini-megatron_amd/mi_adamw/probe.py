@@ -64,9 +64,10 @@ def time_probe(opt, launches: int = 20) -> float | None:
                 _lib.check(lib.mi_adamw_probe_flat(ctypes.byref(row), chunk, state, flags,
                                                    opt.max_blocks, stream), "mi_adamw_probe_flat")
             else:
-                _lib.check(lib.mi_adamw_probe(launch.rows.data_ptr(), launch.chunks.data_ptr(),
-                                              launch.n_chunks, chunk, state, flags,
-                                              opt.max_blocks, stream), "mi_adamw_probe")
+                _lib.check(lib.mi_adamw_probe(launch.rows.data_ptr(), launch.items.data_ptr(),
+                                              launch.n_items, chunk, state,
+                                              flags | launch.item_flag, opt.max_blocks, stream),
+                           "mi_adamw_probe")
 
         events = [(torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True))
                   for _ in range(launches)]

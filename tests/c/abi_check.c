@@ -142,6 +142,11 @@ static int cpu_checks(void)
               "chunk %d", i);
     CHECK(mi_adamw_build_chunks(numels, 5, 1000, NULL, 0) == MI_ADAMW_E_INVALID, "chunk size");
     CHECK(mi_adamw_build_chunks(numels, 5, 4096, chunks, 6) == MI_ADAMW_E_INVALID, "capacity");
+    CHECK(mi_adamw_build_tiles(numels, 5, NULL, 0) == 0 + 1 + 4 + 5 + 12, "tile count");
+    CHECK(mi_adamw_build_tiles(numels, 3, chunks, 7) == 5 && chunks[4].tensor == 2 &&
+              chunks[4].index == 3, "tile fill");
+    CHECK(mi_adamw_build_tiles(numels, 5, chunks, 7) == MI_ADAMW_E_INVALID, "tile capacity");
+    CHECK(mi_adamw_build_tiles(NULL, 5, NULL, 0) == MI_ADAMW_E_INVALID, "tiles of nothing");
 
     /* Every call below is refused on the host before anything is launched. */
     mi_adamw_hyper h[1];
@@ -190,6 +195,13 @@ static int cpu_checks(void)
     CHECK(mi_adamw_step_capturable_rows(fake, 0, fake, 1, 4096, &ch, 1, fake, fake,
                                         (void *)(uintptr_t)4096, NULL, 0, 0, 0, NULL) ==
               MI_ADAMW_E_INVALID, "capturable rows with no rows");
+    CHECK(mi_adamw_step_capturable(fake, fake, 1, 4096, &ch, 1, fake, fake, NULL, 0,
+                                   MI_ADAMW_F_TILES, 0, NULL) == MI_ADAMW_E_INVALID,
+          "tiles where a workgroup takes 4096 elements");
+    CHECK(mi_adamw_step_flat(&t, h, NULL, 4096, MI_ADAMW_STATE_F32, MI_ADAMW_F_TILES, 0, NULL) ==
+              MI_ADAMW_E_INVALID, "tiles of a flat range");
+    CHECK(mi_adamw_probe_flat(&t, 4096, MI_ADAMW_STATE_F32, MI_ADAMW_F_TILES, 0, NULL) ==
+              MI_ADAMW_E_INVALID, "probe of a flat range's tiles");
     CHECK(mi_adamw_widen_bf16(NULL, fake, 1, 4096, NULL) == MI_ADAMW_E_INVALID,
           "widen without tensors");
     CHECK(mi_adamw_widen_bf16(fake, fake, 0, 4096, NULL) == MI_ADAMW_E_INVALID,
