@@ -901,7 +901,8 @@ struct Tile {
     }
 };
 
-constexpr int kUpdRun = 128;
+constexpr int kUpdTile = MI_ADAMW_TILE_ELEMS;   // of 256 lanes
+constexpr int kUpdRun = 128;                    // in tiles of kUpdTile elements
 
 // Lanes of an instance's workgroups.  The chains whose first wave forms the per-step
 // values for the whole workgroup (kShare: a few hundred instructions) take the widest
@@ -945,9 +946,19 @@ __device__ __forceinline__ typename HS::Scalars shared_scalars(const HS& hs,
 // mi_adamw_norm_block (block_coef).
 enum Clip { kNoClip, kCoef, kBlock };
 
+// Waves per SIMD: four, the cap above, with 128 VGPRs per lane.  The 1024-lane workgroups
+// whose barrier waits for the first wave take eight, two per CU, so that one computes while
+// the other waits, where 64 VGPRs suffice.  mi_adamw_step_capturable in us, with four waves
+// (and runs of 128 workgroups) and with eight: 2,000 tensors of 768 elements 21.5 and 14.2,
+// 300 of them 6.5 and 4.9, 5M parameters 22.6 and 20.7, 17M 68.2 and 66.9, 124M 560 and 584.
+template <class HS, Clip kClip, bool kAms>
+constexpr int update_waves() {
+    return HS::kShare && kClip != kBlock && !kAms ? 8 : 4;
+}
+
 template <class Src, class HS, typename StateT, Clip kClip, bool kCopy, bool kWriteGrad, bool kAms>
 __global__ __launch_bounds__(update_threads<HS>())
-__attribute__((amdgpu_waves_per_eu(4, 4)))   // the cap above, and 128 VGPRs per lane
+__attribute__((amdgpu_waves_per_eu(update_waves<HS, kClip, kAms>(), update_waves<HS, kClip, kAms>())))
 void mi_adamw_update_kernel(
     Src src, Items items, HS hs, const float* __restrict__ grad_scale, float pre) {
     using IO = StateIO<StateT>;
@@ -970,7 +981,8 @@ void mi_adamw_update_kernel(
         mi_adamw_tensor t;
         int64_t begin, end;
         int32_t row;
-        if (!items.get<kTile>(src, item_order<kUpdRun>(w, items.n), t, begin, end, row)) continue;
+        const int64_t it = item_order<kUpdRun * kUpdTile / kTile>(w, items.n);
+        if (!items.get<kTile>(src, it, t, begin, end, row)) continue;
         // Default chain: the scalars are kernel arguments.  Capturable and fused
         // chains: they are formed once the tile's loads are in flight; in the
         // capturable chain (two powf, three divisions: a few hundred instructions) by
