@@ -951,8 +951,11 @@ enum Clip { kNoClip, kCoef, kBlock };
 // the other waits, where 64 VGPRs suffice.  mi_adamw_step_capturable in us, with four waves
 // (and runs of 128 workgroups) and with eight: 2,000 tensors of 768 elements 21.5 and 14.2,
 // 300 of them 6.5 and 4.9, 5M parameters 22.6 and 20.7, 17M 68.2 and 66.9, 124M 560 and 584.
+// Where every wave forms them by two float64 pow (the fused=True chain at device step
+// counts), six hide more of that and still hold 80 VGPRs: 17M 85.1 and 79.8, 124M 688 and 652.
 template <class HS, Clip kClip, bool kAms>
 constexpr int update_waves() {
+    if (std::is_same<HS, FusedHyper<true>>::value) return 6;
     return HS::kShare && kClip != kBlock && !kAms ? 8 : 4;
 }
 
