@@ -299,10 +299,9 @@ int mi_adamw_norm_from_sumsq(const double *d_sumsq, int32_t n, float max_norm, f
 
 /* New gradient pointers for rows of a device tensor table of n_rows rows: row rows[i]
  * gets grads[i], and its MI_ADAMW_T_VEC flag set if vec[i] is non-zero, cleared if not
- * (the caller sets vec[i] when every pointer of the row, the new gradient included, is
- * aligned for the vector path).  For the step after zero_grad() freed the gradients and
- * backward allocated new ones (main.py:204-209): only the gradient column of the table
- * changes.  rows, grads and vec are host arrays of n entries, carried to the device as
+ * (the flag's promise covers every pointer of the row, the new gradient included).  For
+ * the step after zero_grad() freed the gradients and backward allocated new ones
+ * (main.py:204-209): only the gradient column of the table changes.  rows, grads and vec are host arrays of n entries, carried to the device as
  * kernel arguments, so they may be reused as soon as the call returns.  Each row may
  * appear at most once (MI_ADAMW_E_INVALID otherwise, as for a row outside [0, n_rows)).
  * Ordered on the stream like every other call: launches queued earlier on it still see
@@ -323,8 +322,7 @@ int mi_adamw_scale_grads(const mi_adamw_tensor *d_tensors, const mi_adamw_chunk 
  * mini-megatron's --amp forward (main.py:93; F.linear at
  * parallel/tensor_parallel.py:55,79), which widens each bf16 weight gradient for its
  * fp32 master.  mi_adamw.bf16_weights, which replaces the forward cast, widens all
- * of them with this one launch.  MI_ADAMW_T_VEC: param 16-byte and param_copy 8-byte
- * aligned. */
+ * of them with this one launch. */
 int mi_adamw_widen_bf16(const mi_adamw_tensor *d_tensors, const mi_adamw_chunk *d_chunks,
                         int64_t n_chunks, int64_t chunk_elems, void *stream);
 

@@ -91,7 +91,7 @@ struct Entry {
     int32_t row = kNoRow;       // table row to patch, or kNoRow / kFixed
     int32_t slot = 0;           // index into the step buffer
     int32_t hyper = 0;          // hyperparameter set (one per param group)
-    uint8_t rest = 0;           // the row's other pointers are aligned for the vector path
+    uint8_t rest = 0;           // the row's other pointers keep MI_ADAMW_T_VEC's promise
 };
 
 struct Plan {
@@ -191,7 +191,9 @@ PyObject* py_bind(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
 //   launch:          (tables, d_rows, d_chunks, n_chunks, n_rows, host_rows, flat_row_addr,
 //                     flat_hyper)
 //   options:         (chunk_elems, max_blocks, state_code, flags, clip, max_norm, prescale,
-//                     norm_block, grad_scale, 0, stream, fused_chain[, d_items, n_items])
+//                     norm_block, grad_scale, 0, stream, fused_chain[, d_items, n_items]);
+//                     grad_scale: what the update takes as its gradient scale, the norm
+//                     block; the 0 is not read; d_items: the update's table, if not d_chunks
 //   keep:            objects to keep alive while the plan exists
 PyObject* plan_new(PyObject* args);
 

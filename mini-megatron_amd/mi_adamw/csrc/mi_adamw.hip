@@ -26,8 +26,8 @@
 //                          arithmetic, values stored back unchanged (a measurement twin).
 //
 // Every launch walks a chunk table (one entry per `chunk_elems` slice of a
-// tensor) so that all parameter tensors go through one launch, or one
-// contiguous range in the flat-buffer layout.
+// tensor; an update also a table of its tiles) so that all parameter tensors go
+// through one launch, or one contiguous range in the flat-buffer layout.
 //
 // The default element math follows torch's per-op chain (torch/optim/adam.py:419-547)
 // with one fp32 rounding per ATen op; the fused=True chain follows adam_math of
@@ -1536,7 +1536,7 @@ const char* mi_adamw_version(void) {
 const char* mi_adamw_strerror(int code) {
     if (code == MI_ADAMW_OK) return "success";
     if (code == MI_ADAMW_E_INVALID) return "mi_adamw: invalid argument (size, count or pointer)";
-    if (code == MI_ADAMW_E_ALIGN) return "mi_adamw: pointer not aligned for the vector path";
+    if (code == MI_ADAMW_E_ALIGN) return "mi_adamw: misaligned pointer of a tensor flagged aligned";
     if (code == MI_ADAMW_E_SCRATCH)
         return "mi_adamw: the launch needs more partial sums than the library's static scratch holds";
     if (code > 0) return hipGetErrorString(static_cast<hipError_t>(code));
@@ -1570,7 +1570,6 @@ int mi_adamw_grad_norm_flat(const float* d_grad, int64_t n, int64_t chunk_elems,
     memset(&src.t, 0, sizeof(src.t));
     src.t.grad = const_cast<float*>(d_grad);
     src.t.numel = n;
-    src.t.flags = aligned(d_grad, 16) ? MI_ADAMW_T_VEC : 0;
     const int64_t n_chunks = (n + chunk_elems - 1) / chunk_elems;
     return launch_norm(src, n_chunks, chunk_elems, max_norm, d_partials, d_norm, d_coef,
                        static_cast<hipStream_t>(stream));
@@ -1611,7 +1610,6 @@ int mi_adamw_grad_norm_flat_noalloc(const float* d_grad, int64_t n, int64_t chun
     memset(&src.t, 0, sizeof(src.t));
     src.t.grad = const_cast<float*>(d_grad);
     src.t.numel = n;
-    src.t.flags = aligned(d_grad, 16) ? MI_ADAMW_T_VEC : 0;
     const int64_t n_chunks = (n + chunk_elems - 1) / chunk_elems;
     return launch_norm(src, n_chunks, chunk_elems, max_norm, partials, d_norm, d_coef, s,
                        kScratchDoubles);
@@ -1635,7 +1633,6 @@ int mi_adamw_grad_sumsq_flat(const float* d_grad, int64_t n, int64_t chunk_elems
     memset(&src.t, 0, sizeof(src.t));
     src.t.grad = const_cast<float*>(d_grad);
     src.t.numel = n;
-    src.t.flags = aligned(d_grad, 16) ? MI_ADAMW_T_VEC : 0;
     const int64_t n_chunks = (n + chunk_elems - 1) / chunk_elems;
     return launch_sumsq_total(src, n_chunks, chunk_elems, grad_prescale, d_partials, d_sumsq,
                               static_cast<hipStream_t>(stream));

@@ -317,8 +317,8 @@ class _Fast:
 
 
 class FusedAdamW(Optimizer):
-    """AdamW with the whole step fused into one MI355X kernel launch (three with the
-    global-norm clip: sum of squares, finalize, update).
+    """AdamW with the whole step fused into one MI355X kernel launch (with the
+    global-norm clip three: sum of squares, finalize, update; two for a small set).
 
     The constructor takes torch.optim.AdamW's arguments, with its defaults and
     its ValueError checks (amsgrad and maximize work as in torch).  With
