@@ -17,7 +17,8 @@ moments, in the layouts the optimizer offers) are timed in the same run as rows
 of ``sweep``, each with its own ``roofline``.  Before its timed steps each set
 takes one step and ``FusedAdamW.place_buffers(16)`` (``--placement-trials``): the
 streams the update writes move to the fastest of up to 16 more allocations, by
-the update's memory-only twin; each row's ``placement`` holds that report.
+the update's memory-only twin; each row's ``placement`` sums that report up (stderr has
+all of it, so that the line stays short of the 16,000 characters that a log may keep).
 
 Output: one JSON line.  ``value`` is the achieved HBM bandwidth of the whole
 step in GB/s, from algorithmic bytes (every byte the step must read or write,
@@ -92,6 +93,20 @@ def bytes_per_param(clip: bool, state: str, copy: bool,
 
 def log(msg: str) -> None:
     print(msg, file=sys.stderr, flush=True)
+
+
+def placement_brief(report: dict | None) -> dict | None:
+    """place_buffers' report without each candidate's time: the twin on the first and on the
+    chosen set, and per stream tried (in sweeps) the chosen one of how many."""
+    if report is None:
+        return None
+    keep = ("layout", "candidates", "chosen", "total_twin_gain", "peak_transient_bytes", "seconds",
+            "ab", "later_passes")
+    out = {k: report[k] for k in keep if k in report}
+    out["twin_ms"] = [report["twin_ms"][0], report["twin_ms"][report["chosen"]]]
+    out["per_stream"] = ", ".join(f"{st['stream']} {st['chosen']}/{st['candidates']}"
+                                  for st in report["per_stream"])
+    return out
 
 
 def build_set(name: str, device, capturable: bool = False, write_grads: bool = False):
@@ -589,7 +604,7 @@ def run_config(name: str, steps: int, warmup: int, device, with_context: bool,
         "bytes_per_param": total_b, "bytes_per_step": step_bytes,
         "gbs": step_bytes / gpu_ms / 1e6, "pct_of_peak": 100 * step_bytes / gpu_ms / 1e6 / PEAK_HBM_GBS,
         "params_per_s": n / gpu_ms * 1e3,
-        "placement": placement,
+        "placement": placement_brief(placement),
         "norm_kernel_ms": norm_avg, "update_kernel_ms": upd_avg,
         "update_kernel_ms_p90": _pct(upd_ms, 0.9),
         "step_ms_median": statistics.median(step_ms), "step_ms_p90": _pct(step_ms, 0.9),
@@ -814,7 +829,7 @@ def main() -> int:
             else:
                 for row in line.get("sweep", []):
                     if row["config"] == nm:
-                        row["cpu_baseline"] = cb
+                        row["cpu_baseline"] = {k: v for k, v in cb.items() if k != "host"}
     print(json.dumps(line), flush=True)
     return 0
 
