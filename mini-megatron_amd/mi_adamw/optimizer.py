@@ -1147,15 +1147,15 @@ class FusedAdamW(Optimizer):
             return self._flat_rows(entries, hyper_idx, ams)
         return self._tensor_rows(entries, hyper_idx, ams)
 
-    def _new_launch(self, entries, hyper_idx, ams, device) -> _Launch:
+    def _new_launch(self, entries, hyper_idx, ams, device, update: bool = True) -> _Launch:
         if self.capturable:
             # one row per tensor (each has its own device step count), always as tables
             rows, src, rest = self._tensor_rows(entries, hyper_idx, ams)
             slots = np.asarray([entries[i][0].slot for i in src], dtype=np.int32)
             return _Launch(rows, self.chunk_elems, device, tables=True, src=src, rest=rest,
-                           step_slots=slots, update=True)
+                           step_slots=slots, update=update)
         rows, src, rest = self._rows(entries, hyper_idx, ams)
-        return _Launch(rows, self.chunk_elems, device, src=src, rest=rest, update=True)
+        return _Launch(rows, self.chunk_elems, device, src=src, rest=rest, update=update)
 
     def _flat_rows(self, entries, hyper_idx, ams):
         """One row per param group whose every param steps with one hyper set."""
@@ -1316,7 +1316,8 @@ class FusedAdamW(Optimizer):
             if len(parts) == 1:
                 norm_launch = launches[0]
             else:
-                norm_launch = self._new_launch(entries, [0] * len(entries), False, device)
+                norm_launch = self._new_launch(entries, [0] * len(entries), False, device,
+                                               update=False)
             self._launch_cache = _LaunchCache(sig, device, launches, norm_launch, grads)
 
         ev = self.timing_events

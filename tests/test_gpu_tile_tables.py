@@ -67,6 +67,8 @@ def test_tiles_give_the_bits_of_chunks(dev, monkeypatch, opts, groups, chunk):
     for odd in (0, 1):
         got, flags, opt = _run(dev, dict(opts, chunk_elems=chunk), groups, odd)
         assert set(flags) == {_lib.F_TILES}
+        cache = opt._launch_cache
+        assert cache.norm_launch is cache.launches[0] or cache.norm_launch.item_flag == 0
         if groups == 1:
             assert time_probe(opt, launches=2) > 0.0     # the twin of this launch
         with monkeypatch.context() as m:
